@@ -430,24 +430,7 @@ __global__ __launch_bounds__(512) void k_gemm_big(const uint8_t *__restrict__ A,
         for (int i = 0; i < 4; ++i) ar[i] = sA + (wm * 128 + i * 32 + l32) * LDS_STRIDE;
 #pragma unroll
         for (int j = 0; j < 2; ++j) br[j] = sB + (wn * 64 + j * 32 + l32) * LDS_STRIDE;
-        if constexpr (PREC == MTIP_FP32) {
-#pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                const int off = g * 32 + half * 16;
-                floatx4 av[4], bv[2];
-#pragma unroll
-                for (int i = 0; i < 4; ++i) av[i] = *(const floatx4 *)(ar[i] + off);
-#pragma unroll
-                for (int j = 0; j < 2; ++j) bv[j] = *(const floatx4 *)(br[j] + off);
-#pragma unroll
-                for (int t = 0; t < 4; ++t)
-#pragma unroll
-                    for (int i = 0; i < 4; ++i)
-#pragma unroll
-                        for (int j = 0; j < 2; ++j)
-                            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(av[i][t], bv[j][t], acc[i][j], 0, 0, 0);
-            }
-        } else if constexpr (PREC == MTIP_BF16) {
+        if constexpr (PREC == MTIP_BF16) {
             // fragments of sub-step s4 + 1 are read while sub-step s4's MFMAs run
             bf16x8 av[2][4], bv[2][2];
             auto frag = [&](int s4, int b) __attribute__((always_inline)) {
@@ -581,6 +564,309 @@ __global__ __launch_bounds__(512) void k_gemm_big(const uint8_t *__restrict__ A,
 #pragma unroll
                 for (int r = 0; r < K; ++r) dst[r] = top[bn][r];
             }
+        }
+    }
+}
+
+// ---------------------------------------------------------------- FP32 cross term
+//
+// FP32 operands on the bf16 matrix instructions: every FP32 value is the exact
+// sum of three bf16 values (8 + 8 + 8 bits, each the rounding of what the ones
+// before leave), split while a stage goes from registers to LDS.  Of the nine
+// partial products the six of relative size 2^-16 and above are accumulated in
+// FP32; the three left out are below 2^-25 of |a b|, half an FP32 rounding.
+// The bf16 instructions run 16 times the FP32 ones' rate, so six of them cost
+// 6 / 16 of the FP32 product's time, and a sum takes 6 roundings per 16 pixels
+// instead of 16: the error against 64 bits is 0.6 - 0.9 of the FP32 instructions'
+// (16 to 16,384 pixels, normal, uniform and centred photon data; equal on data
+// of a wide range).  10,000 x 10,000 x 16,384: 26.8 -> 16.2 ms.  A tile whose sums are not all finite (an infinity or a NaN in an
+// operand, a sum beyond FP32) is computed again with the FP32 instructions, so
+// such values rank as they do there.
+//
+// A workgroup of 2 x WN waves owns a tile of 64 NI orientations x 64 WN images
+// (256 x 256 or 128 x 128), each wave NI x 2 blocks of 32 x 32.  K goes in stages
+// of 16 pixels, double-buffered: a staged row is 3 x 32 bytes and 16 more that
+// spread 16 rows over the banks.
+constexpr int kSplitK = 16;
+constexpr int kSplitRow = 3 * 2 * kSplitK + 16;
+
+typedef float floatx2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+
+// w[p] (p = 0, 1, 2): the p-th bf16 parts of a pair of floats
+__device__ __forceinline__ void split_pair(float a, float b, uint32_t (&w)[3])
+{
+#pragma unroll
+    for (int p = 0; p < 3; ++p) {
+        const uint32_t h = __builtin_bit_cast(uint32_t, __builtin_convertvector((floatx2{a, b}), bf16x2));
+        w[p] = h;
+        a -= __uint_as_float(h << 16);
+        b -= __uint_as_float(h & 0xffff0000u);
+    }
+}
+
+//
+// Top-K keys come per `rows` orientations: 64 NI, or (HALVES) 32 NI, the rows of
+// one wave, so that the 256-row tile can fill the layout of the 128-row one.
+// Workgroups [0, nwa nwb) take the whole tiles, those after them the thin ones
+// of the last row or column (edge_plan), whose waves skip the blocks without a
+// valid row or column: they end the launch with a short round instead of
+// sharing a full one.
+template <int NI, int WN, int K, bool HALVES>
+__global__ __launch_bounds__(128 * WN) void k_gemm_split(
+    const float *__restrict__ A, int64_t lda, int64_t NA, const float *__restrict__ B, int64_t ldb,
+    int64_t NB, int n_pix, const double *__restrict__ sumsqA, const double *__restrict__ alpha,
+    int nta, int ntb, int nwa, int nwb, int n_key_tiles, uint64_t *__restrict__ part)
+{
+    constexpr int TM = 64 * NI, TN = 64 * WN, NT = 128 * WN;
+    constexpr int STAGE = (TM + TN) * kSplitRow;
+    constexpr int PLAIN = (TM + TN) * LDS_STRIDE;       // a stage of the FP32 instructions
+    __shared__ __attribute__((aligned(16))) uint8_t smem[2 * STAGE > PLAIN ? 2 * STAGE : PLAIN];
+    __shared__ float s_rowc[TM];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm = wave & 1, wn = wave >> 1;
+    const int half = lane >> 5, l32 = lane & 31;
+    int ta, tb;
+    const bool thin = (int)blockIdx.x >= nwa * nwb;
+    if (!thin) {
+        tile_of(blockIdx.x, nwa * nwb, nwa, nwb, ta, tb);
+    } else {
+        const int t = (int)blockIdx.x - nwa * nwb, n_row = nwa < nta ? ntb : 0;
+        ta = t < n_row ? nta - 1 : t - n_row;
+        tb = t < n_row ? t : ntb - 1;
+    }
+    const int64_t a0 = (int64_t)ta * TM, b0 = (int64_t)tb * TN;
+    for (int i = tid; i < TM; i += NT) {
+        const int64_t r = a0 + i;
+        const double al = *alpha;
+        s_rowc[i] = r < NA ? (float)(al * al * sumsqA[r]) : 0.0f;
+    }
+    floatx16 acc[NI][2];
+    auto clear = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < NI; ++i)
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+#pragma unroll
+                for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.0f;
+    };
+    clear();
+    typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+    const int rowsA = (int)min((int64_t)TM, NA - a0), rowsB = (int)min((int64_t)TN, NB - b0);
+    const __amdgpu_buffer_rsrc_t rsA = __builtin_amdgcn_make_buffer_rsrc(
+        (void *)(A + a0 * lda), (short)0, (int)((int64_t)rowsA * lda * 4), 0x00020000);
+    const __amdgpu_buffer_rsrc_t rsB = __builtin_amdgcn_make_buffer_rsrc(
+        (void *)(B + b0 * ldb), (short)0, (int)((int64_t)rowsB * ldb * 4), 0x00020000);
+    // staging: thread t takes 8 pixels (t & 1) of row t >> 1 (+ NT / 2) of the
+    // tile's TM rows of A, then TN rows of B
+    static_assert(TM == TN && (TM + TN) * 2 == 2 * NT, "one A and one B row half per thread");
+    const int r_st = tid >> 1, h_st = tid & 1;
+    const int vA = (r_st * (int)lda + 8 * h_st) * 4, vB = (r_st * (int)ldb + 8 * h_st) * 4;
+    const int n_stages = (n_pix + kSplitK - 1) / kSplitK;     // loads past it read zeros
+    u32x4 ra[2], rb[2];
+    auto load_stage = [&](int st) __attribute__((always_inline)) {
+        const bool in_k = st < n_stages;
+        const int oa = in_k ? vA + st * (kSplitK * 4) : 0x7fffffe0;
+        const int ob = in_k ? vB + st * (kSplitK * 4) : 0x7fffffe0;
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            ra[i] = __builtin_amdgcn_raw_buffer_load_b128(rsA, oa + 16 * i, 0, 0);
+            rb[i] = __builtin_amdgcn_raw_buffer_load_b128(rsB, ob + 16 * i, 0, 0);
+        }
+    };
+    auto store_half = [&](uint8_t *dst, const u32x4 (&r)[2]) __attribute__((always_inline)) {
+        u32x4 w[3];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            uint32_t p[3];
+            split_pair(__uint_as_float(r[e >> 1][2 * (e & 1)]), __uint_as_float(r[e >> 1][2 * (e & 1) + 1]), p);
+#pragma unroll
+            for (int q = 0; q < 3; ++q) w[q][e] = p[q];
+        }
+#pragma unroll
+        for (int q = 0; q < 3; ++q) *(u32x4 *)(dst + q * 32) = w[q];
+    };
+    auto store_stage = [&](int buf) __attribute__((always_inline)) {
+        uint8_t *d = smem + buf * STAGE + r_st * kSplitRow + 16 * h_st;
+        store_half(d, ra);
+        store_half(d + TM * kSplitRow, rb);
+    };
+
+    // blocks of 32 this wave has valid rows and columns for
+    const int vi = min(NI, max(0, (rowsA - wm * 32 * NI + 31) >> 5));
+    const int vj = min(2, max(0, (rowsB - wn * 64 + 31) >> 5));
+    load_stage(0);
+    store_stage(0);
+    load_stage(1);
+    __syncthreads();
+    // the small products first
+    constexpr int pa[6] = {2, 0, 1, 1, 0, 0}, pb[6] = {0, 2, 1, 0, 1, 0};
+    auto frag = [](const uint8_t *p, bf16x8 (&v)[3]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int q = 0; q < 3; ++q) v[q] = *(const bf16x8 *)(p + q * 32);
+    };
+    const uint8_t *const sA0 = smem + (wm * 32 * NI + l32) * kSplitRow + 16 * half;
+    const uint8_t *const sB0 = smem + (TM + wn * 64 + l32) * kSplitRow + 16 * half;
+    if (!thin) {
+        for (int st = 0; st < n_stages; ++st) {
+            const int buf = st & 1;
+            store_stage(buf ^ 1);
+            load_stage(st + 2);
+            bf16x8 bv[2][3];
+            frag(sB0 + buf * STAGE, bv[0]);
+            frag(sB0 + buf * STAGE + 32 * kSplitRow, bv[1]);
+#pragma unroll
+            for (int i = 0; i < NI; ++i) {
+                bf16x8 av[3];
+                frag(sA0 + buf * STAGE + i * 32 * kSplitRow, av);
+#pragma unroll
+                for (int t = 0; t < 6; ++t)
+#pragma unroll
+                    for (int j = 0; j < 2; ++j)
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av[pa[t]], bv[j][pb[t]], acc[i][j], 0, 0, 0);
+            }
+            // The small tile (4000 x 2000 x 16,384: 1.57 -> 1.43 ms): each MFMA
+            // followed by the next block's fragment reads, then two of the split's
+            // instructions, and the staging at the end.  The large one is held by
+            // its power draw (1.6 GHz at 71 % matrix-core busy), and the same
+            // order costs it 4 %
+            if constexpr (NI == 2) {
+                __builtin_amdgcn_sched_group_barrier(0x100, 9, 0);
+#pragma unroll
+                for (int m = 0; m < 12 * NI; ++m) {
+                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                    if (m % 12 < 3 && m < 12 * (NI - 1)) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+                    __builtin_amdgcn_sched_group_barrier(0x002, 2, 0);
+                    if ((m >= 6 * NI - 2 && m < 6 * NI + 1) || m >= 12 * NI - 4)
+                        __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);
+                    if (m >= 12 * NI - 4) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
+                }
+            }
+            __syncthreads();
+        }
+    } else {
+        for (int st = 0; st < n_stages; ++st) {
+            const int buf = st & 1;
+            store_stage(buf ^ 1);
+            load_stage(st + 2);
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                if (j < vj && vi > 0) {
+                    bf16x8 bv[3];
+                    frag(sB0 + buf * STAGE + j * 32 * kSplitRow, bv);
+#pragma unroll
+                    for (int i = 0; i < NI; ++i) {
+                        if (i < vi) {
+                            bf16x8 av[3];
+                            frag(sA0 + buf * STAGE + i * 32 * kSplitRow, av);
+#pragma unroll
+                            for (int t = 0; t < 6; ++t)
+                                acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av[pa[t]], bv[pb[t]], acc[i][j], 0, 0, 0);
+                        }
+                    }
+                }
+            }
+            __syncthreads();
+        }
+    }
+    // infinities and NaN: this tile again, plainly
+    bool fine = true;
+#pragma unroll
+    for (int i = 0; i < NI; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) fine &= fabsf(acc[i][j][v]) <= 3.402823466e38f;
+    if (__syncthreads_or(!fine)) {
+        clear();
+        constexpr int PK = 32;      // pixels a stage
+        for (int k0 = 0; k0 < n_pix; k0 += PK) {
+            for (int c = tid; c < (TM + TN) * (PK / 4); c += NT) {
+                const int r = c / (PK / 4), col = k0 + 4 * (c % (PK / 4));
+                const bool in_k = col < n_pix;
+                const u32x4 v = r < TM
+                    ? __builtin_amdgcn_raw_buffer_load_b128(rsA, in_k ? (r * (int)lda + col) * 4 : 0x7fffffe0, 0, 0)
+                    : __builtin_amdgcn_raw_buffer_load_b128(rsB, in_k ? ((r - TM) * (int)ldb + col) * 4 : 0x7fffffe0, 0, 0);
+                *(u32x4 *)(smem + r * LDS_STRIDE + 16 * (c % (PK / 4))) = v;
+            }
+            __syncthreads();
+            for (int g = 0; g < PK / 8; ++g) {
+                const int off = g * 32 + half * 16;
+                floatx4 av[NI], bv[2];
+#pragma unroll
+                for (int i = 0; i < NI; ++i)
+                    av[i] = *(const floatx4 *)(smem + (wm * 32 * NI + i * 32 + l32) * LDS_STRIDE + off);
+#pragma unroll
+                for (int j = 0; j < 2; ++j)
+                    bv[j] = *(const floatx4 *)(smem + (TM + wn * 64 + j * 32 + l32) * LDS_STRIDE + off);
+#pragma unroll
+                for (int t = 0; t < 4; ++t)
+#pragma unroll
+                    for (int i = 0; i < NI; ++i)
+#pragma unroll
+                        for (int j = 0; j < 2; ++j)
+                            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(av[i][t], bv[j][t], acc[i][j], 0, 0, 0);
+            }
+            __syncthreads();
+        }
+    }
+
+    // per image column the K smallest v over the tile's rows
+    const float two_a = 2.0f * (float)(*alpha);
+    uint64_t top[2][K];
+#pragma unroll
+    for (int bn = 0; bn < 2; ++bn) {
+#pragma unroll
+        for (int r = 0; r < K; ++r) top[bn][r] = KEY_NONE;
+#pragma unroll
+        for (int bm = 0; bm < NI; ++bm) {
+#pragma unroll
+            for (int v = 0; v < 16; ++v) {
+                const int m = wm * 32 * NI + bm * 32 + 8 * (v >> 2) + 4 * half + (v & 3);
+                const int64_t go = a0 + m;
+                if (go < NA) {
+                    const float val = fmaf(-two_a, acc[bm][bn][v], s_rowc[m]);
+                    mtip::topk_insert<K>(top[bn], mtip::make_key(val, (uint32_t)go));
+                }
+            }
+        }
+        uint64_t other[K];
+#pragma unroll
+        for (int r = 0; r < K; ++r) other[r] = mtip::shfl_xor_u64(top[bn][r], 32);
+        mtip::topk_merge<K>(top[bn], other);
+    }
+    auto put = [&](int bn, int key_tile) __attribute__((always_inline)) {
+        const int64_t gi = b0 + wn * 64 + bn * 32 + l32;
+        if (gi < NB && key_tile < n_key_tiles) {
+            uint64_t *dst = part + (gi * n_key_tiles + key_tile) * K;
+#pragma unroll
+            for (int r = 0; r < K; ++r) dst[r] = top[bn][r];
+        }
+    };
+    if constexpr (HALVES) {
+        if (half == 0) {
+            put(0, 2 * ta + wm);
+            put(1, 2 * ta + wm);
+        }
+        return;
+    }
+    uint64_t *s_top = (uint64_t *)smem;    // [WN][64 cols][K] (after the last barrier)
+    if (wm == 1 && half == 0) {
+#pragma unroll
+        for (int bn = 0; bn < 2; ++bn)
+#pragma unroll
+            for (int r = 0; r < K; ++r) s_top[(wn * 64 + bn * 32 + l32) * K + r] = top[bn][r];
+    }
+    __syncthreads();
+    if (wm == 0 && half == 0) {
+#pragma unroll
+        for (int bn = 0; bn < 2; ++bn) {
+            uint64_t other[K];
+#pragma unroll
+            for (int r = 0; r < K; ++r) other[r] = s_top[(wn * 64 + bn * 32 + l32) * K + r];
+            mtip::topk_merge<K>(top[bn], other);
+            put(bn, ta);
         }
     }
 }
@@ -1116,13 +1402,45 @@ size_t edge_bytes(int64_t N_o, int64_t N_i)
     return (size_t)p.n_thin * p.splits * p.slot * sizeof(float);
 }
 
+// FP32: 256 x 256 tiles of k_gemm_split once there is most of a round of them,
+// whatever the rows per key tile (the keys do not depend on it), else 128 x 128.
+template <int K>
+void launch_split_topk(const float *S, int64_t lds, int64_t N_o, const float *D, int64_t ldd,
+                       int64_t N_i, int n_pix, const double *s2, const double *alpha, int tile,
+                       uint64_t *part, hipStream_t st)
+{
+    const EdgePlan p = edge_plan(N_o, N_i);
+    const int n_key = (int)mtip::ceil_div(N_o, tile);
+    const dim3 grid((unsigned)(p.nwa * p.nwb + p.n_thin));
+    if (tile == BM2) {
+        hipLaunchKernelGGL((k_gemm_split<4, 4, K, false>), grid, dim3(512), 0, st, S, lds, N_o, D,
+                           ldd, N_i, n_pix, s2, alpha, p.nta, p.ntb, p.nwa, p.nwb, n_key, part);
+    } else if (p.nta * p.ntb >= 192 && (int64_t)BM2 * std::max(lds, ldd) * 4 < ((int64_t)1 << 31)) {
+        hipLaunchKernelGGL((k_gemm_split<4, 4, K, true>), grid, dim3(512), 0, st, S, lds, N_o, D,
+                           ldd, N_i, n_pix, s2, alpha, p.nta, p.ntb, p.nwa, p.nwb, n_key, part);
+    } else {
+        const int nta = (int)mtip::ceil_div(N_o, BM), ntb = (int)mtip::ceil_div(N_i, BN);
+        hipLaunchKernelGGL((k_gemm_split<2, 2, K, false>), dim3((unsigned)(nta * ntb)), dim3(256), 0,
+                           st, S, lds, N_o, D, ldd, N_i, n_pix, s2, alpha, nta, ntb, nta, ntb,
+                           n_key, part);
+    }
+}
+
 template <int PREC, int K>
 void launch_gemm_topk(const void *S, int64_t lds_b, int64_t N_o, const void *D, int64_t ldd_b,
                       int64_t N_i, int64_t kbytes, const float *ssc, const float *dsc,
                       const double *s2, const double *alpha, int tile, uint64_t *part,
                       float *edge_ws, hipStream_t st)
 {
-    if (tile == BM2) {
+    // k_gemm_split addresses a tile's rows with 32-bit buffer offsets (longer
+    // rows, 16 MiB, take the FP32 instructions)
+    if constexpr (PREC == MTIP_FP32) {
+        if ((int64_t)BM * std::max(lds_b, ldd_b) < ((int64_t)1 << 31)) {
+            launch_split_topk<K>((const float *)S, lds_b / 4, N_o, (const float *)D, ldd_b / 4, N_i,
+                                 (int)(kbytes / 4), s2, alpha, tile, part, st);
+            return;
+        }
+    } else if (tile == BM2) {
         EdgePlan p = edge_plan(N_o, N_i);
         if (!edge_ws || !p.n_thin) {
             p.nwa = p.nta;
@@ -1142,12 +1460,12 @@ void launch_gemm_topk(const void *S, int64_t lds_b, int64_t N_o, const void *D, 
                                edge_ws, p.splits, p.slot, p.nta, p.ntb, p.nwa, N_o, N_i, ssc, dsc,
                                s2, alpha, part);
         }
-    } else {
-        const int nta = (int)mtip::ceil_div(N_o, BM), ntb = (int)mtip::ceil_div(N_i, BN);
-        hipLaunchKernelGGL((k_gemm<PREC, K, OUT_TOPK>), dim3((unsigned)(nta * ntb)), dim3(256), 0,
-                           st, (const uint8_t *)S, lds_b, N_o, (const uint8_t *)D, ldd_b, N_i,
-                           kbytes, ssc, dsc, s2, alpha, nta, part, nullptr, (int64_t)0);
+        return;
     }
+    const int nta = (int)mtip::ceil_div(N_o, BM), ntb = (int)mtip::ceil_div(N_i, BN);
+    hipLaunchKernelGGL((k_gemm<PREC, K, OUT_TOPK>), dim3((unsigned)(nta * ntb)), dim3(256), 0, st,
+                       (const uint8_t *)S, lds_b, N_o, (const uint8_t *)D, ldd_b, N_i, kbytes, ssc,
+                       dsc, s2, alpha, nta, part, nullptr, (int64_t)0);
 }
 
 // Indices of the K smallest entries of each row for any K: one workgroup per
