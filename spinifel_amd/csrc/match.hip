@@ -583,8 +583,10 @@ __global__ __launch_bounds__(512) void k_gemm_big(const uint8_t *__restrict__ A,
 // operand, a sum beyond FP32) is computed again with the FP32 instructions, so
 // such values rank as they do there.
 //
-// A workgroup of 2 x WN waves owns a tile of 64 NI orientations x 64 WN images
-// (256 x 256 or 128 x 128), each wave NI x 2 blocks of 32 x 32.  K goes in stages
+// A workgroup of WM x WN waves owns a tile of 32 NI WM orientations x 64 WN images,
+// each wave NI x 2 blocks of 32 x 32: 256 x 256 in 2 x 4 waves of 128 x 64, 128 x
+// 128 in 2 x 2 waves of 64 x 64, or 128 x 128 in 4 x 2 waves of 32 x 64.  All three
+// add in the same order, so their keys are the same bits.  K goes in stages
 // of 16 pixels, double-buffered: a staged row is 3 x 32 bytes and 16 more that
 // spread 16 rows over the banks.
 constexpr int kSplitK = 16;
@@ -606,29 +608,29 @@ __device__ __forceinline__ void split_pair(float a, float b, uint32_t (&w)[3])
 }
 
 //
-// Top-K keys come per `rows` orientations: 64 NI, or (HALVES) 32 NI, the rows of
-// one wave, so that the 256-row tile can fill the layout of the 128-row one.
+// Top-K keys come per tile of orientations or (HALVES) per 32 NI, the rows of one
+// wave, so that the 256-row tile can fill the layout of the 128-row one.
 // Workgroups [0, nwa nwb) take the whole tiles, those after them the thin ones
 // of the last row or column (edge_plan), whose waves skip the blocks without a
 // valid row or column: they end the launch with a short round instead of
 // sharing a full one.
-template <int NI, int WN, int K, bool HALVES>
-__global__ __launch_bounds__(128 * WN) void k_gemm_split(
+template <int NI, int WM, int WN, int K, bool HALVES>
+__global__ __launch_bounds__(64 * WM * WN) void k_gemm_split(
     const float *__restrict__ A, int64_t lda, int64_t NA, const float *__restrict__ B, int64_t ldb,
     int64_t NB, int n_pix, const double *__restrict__ sumsqA, const double *__restrict__ alpha,
     int nta, int ntb, int nwa, int nwb, int n_key_tiles, uint64_t *__restrict__ part)
 {
-    constexpr int TM = 64 * NI, TN = 64 * WN, NT = 128 * WN;
+    constexpr int TM = 32 * NI * WM, TN = 64 * WN, NT = 64 * WM * WN;
     constexpr int STAGE = (TM + TN) * kSplitRow;
     constexpr int PLAIN = (TM + TN) * LDS_STRIDE;       // a stage of the FP32 instructions
     __shared__ __attribute__((aligned(16))) uint8_t smem[2 * STAGE > PLAIN ? 2 * STAGE : PLAIN];
     __shared__ float s_rowc[TM];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wm = wave & 1, wn = wave >> 1;
+    const int wm = wave % WM, wn = wave / WM;
     const int half = lane >> 5, l32 = lane & 31;
     int ta, tb;
-    const bool thin = (int)blockIdx.x >= nwa * nwb;
+    const bool thin = NI == 4 && (int)blockIdx.x >= nwa * nwb;
     if (!thin) {
         tile_of(blockIdx.x, nwa * nwb, nwa, nwb, ta, tb);
     } else {
@@ -658,21 +660,29 @@ __global__ __launch_bounds__(128 * WN) void k_gemm_split(
         (void *)(A + a0 * lda), (short)0, (int)((int64_t)rowsA * lda * 4), 0x00020000);
     const __amdgpu_buffer_rsrc_t rsB = __builtin_amdgcn_make_buffer_rsrc(
         (void *)(B + b0 * ldb), (short)0, (int)((int64_t)rowsB * ldb * 4), 0x00020000);
-    // staging: thread t takes 8 pixels (t & 1) of row t >> 1 (+ NT / 2) of the
-    // tile's TM rows of A, then TN rows of B
-    static_assert(TM == TN && (TM + TN) * 2 == 2 * NT, "one A and one B row half per thread");
-    const int r_st = tid >> 1, h_st = tid & 1;
-    const int vA = (r_st * (int)lda + 8 * h_st) * 4, vB = (r_st * (int)ldb + 8 * h_st) * 4;
-    const int n_stages = (n_pix + kSplitK - 1) / kSplitK;     // loads past it read zeros
-    u32x4 ra[2], rb[2];
-    auto load_stage = [&](int st) __attribute__((always_inline)) {
-        const bool in_k = st < n_stages;
-        const int oa = in_k ? vA + st * (kSplitK * 4) : 0x7fffffe0;
-        const int ob = in_k ? vB + st * (kSplitK * 4) : 0x7fffffe0;
+    // staging: half rows of 8 pixels, TM rows of A then TN rows of B; thread t takes
+    // halves t + NT i (a wave's are all of one operand)
+    constexpr int kHalves = (TM + TN) * 2 / NT;
+    static_assert(2 * TM % 64 == 0 && (TM + TN) * 2 % NT == 0, "whole waves per operand");
+    const int h_st = tid & 1;
+    int v_st[kHalves];
+    bool of_a[kHalves];
 #pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            ra[i] = __builtin_amdgcn_raw_buffer_load_b128(rsA, oa + 16 * i, 0, 0);
-            rb[i] = __builtin_amdgcn_raw_buffer_load_b128(rsB, ob + 16 * i, 0, 0);
+    for (int i = 0; i < kHalves; ++i) {
+        const int row = (tid + NT * i) >> 1;
+        of_a[i] = (wave * 64 + NT * i) >> 1 < TM;
+        v_st[i] = ((of_a[i] ? row : row - TM) * (int)(of_a[i] ? lda : ldb) + 8 * h_st) * 4;
+    }
+    const int n_stages = (n_pix + kSplitK - 1) / kSplitK;     // loads past it read zeros
+    u32x4 ra[kHalves][2];
+    auto load_stage = [&](int st) __attribute__((always_inline)) {
+        const int ks = st * (kSplitK * 4);
+#pragma unroll
+        for (int i = 0; i < kHalves; ++i) {
+            const int o = st < n_stages ? v_st[i] + ks : 0x7fffffe0;
+            const __amdgpu_buffer_rsrc_t rs = of_a[i] ? rsA : rsB;
+            ra[i][0] = __builtin_amdgcn_raw_buffer_load_b128(rs, o, 0, 0);
+            ra[i][1] = __builtin_amdgcn_raw_buffer_load_b128(rs, o + 16, 0, 0);
         }
     };
     auto store_half = [&](uint8_t *dst, const u32x4 (&r)[2]) __attribute__((always_inline)) {
@@ -688,11 +698,10 @@ __global__ __launch_bounds__(128 * WN) void k_gemm_split(
         for (int q = 0; q < 3; ++q) *(u32x4 *)(dst + q * 32) = w[q];
     };
     auto store_stage = [&](int buf) __attribute__((always_inline)) {
-        uint8_t *d = smem + buf * STAGE + r_st * kSplitRow + 16 * h_st;
-        store_half(d, ra);
-        store_half(d + TM * kSplitRow, rb);
+#pragma unroll
+        for (int i = 0; i < kHalves; ++i)
+            store_half(smem + buf * STAGE + ((tid + NT * i) >> 1) * kSplitRow + 16 * h_st, ra[i]);
     };
-
     // blocks of 32 this wave has valid rows and columns for
     const int vi = min(NI, max(0, (rowsA - wm * 32 * NI + 31) >> 5));
     const int vj = min(2, max(0, (rowsB - wn * 64 + 31) >> 5));
@@ -726,10 +735,10 @@ __global__ __launch_bounds__(128 * WN) void k_gemm_split(
                     for (int j = 0; j < 2; ++j)
                         acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av[pa[t]], bv[j][pb[t]], acc[i][j], 0, 0, 0);
             }
-            // The small tile (4000 x 2000 x 16,384: 1.57 -> 1.43 ms): each MFMA
-            // followed by the next block's fragment reads, then two of the split's
-            // instructions, and the staging at the end.  The large one is held by
-            // its power draw (1.6 GHz at 71 % matrix-core busy), and the same
+            // 128 x 128 in four waves: each MFMA followed by the next block's fragment
+            // reads, then two of the split's instructions, and the staging at the
+            // end (4,000 x 2,000 x 16,384: 1.57 -> 1.50 ms).  The large tile is held
+            // by its power draw (1.6 GHz at 71 % matrix-core busy), and the same
             // order costs it 4 %
             if constexpr (NI == 2) {
                 __builtin_amdgcn_sched_group_barrier(0x100, 9, 0);
@@ -851,21 +860,24 @@ __global__ __launch_bounds__(128 * WN) void k_gemm_split(
         }
         return;
     }
-    uint64_t *s_top = (uint64_t *)smem;    // [WN][64 cols][K] (after the last barrier)
-    if (wm == 1 && half == 0) {
+    uint64_t *s_top = (uint64_t *)smem;    // [WM - 1][TN][K] (after the last barrier)
+    if (wm > 0 && half == 0) {
 #pragma unroll
         for (int bn = 0; bn < 2; ++bn)
 #pragma unroll
-            for (int r = 0; r < K; ++r) s_top[(wn * 64 + bn * 32 + l32) * K + r] = top[bn][r];
+            for (int r = 0; r < K; ++r)
+                s_top[((wm - 1) * TN + wn * 64 + bn * 32 + l32) * K + r] = top[bn][r];
     }
     __syncthreads();
     if (wm == 0 && half == 0) {
 #pragma unroll
         for (int bn = 0; bn < 2; ++bn) {
-            uint64_t other[K];
+            for (int w = 0; w + 1 < WM; ++w) {
+                uint64_t other[K];
 #pragma unroll
-            for (int r = 0; r < K; ++r) other[r] = s_top[(wn * 64 + bn * 32 + l32) * K + r];
-            mtip::topk_merge<K>(top[bn], other);
+                for (int r = 0; r < K; ++r) other[r] = s_top[(w * TN + wn * 64 + bn * 32 + l32) * K + r];
+                mtip::topk_merge<K>(top[bn], other);
+            }
             put(bn, ta);
         }
     }
@@ -1402,8 +1414,12 @@ size_t edge_bytes(int64_t N_o, int64_t N_i)
     return (size_t)p.n_thin * p.splits * p.slot * sizeof(float);
 }
 
-// FP32: 256 x 256 tiles of k_gemm_split once there is most of a round of them,
-// whatever the rows per key tile (the keys do not depend on it), else 128 x 128.
+// FP32: 256 x 256 tiles of k_gemm_split once there is most of a round of them
+// (whatever the rows per key tile: the keys do not depend on it), else 128 x 128.
+// Where those leave a CU with one workgroup or none, its eight waves hide in each
+// other what four do one after the other: split, LDS round trip, products
+// (2,000 x 500 x 1,024 95 -> 78 us, 1,000 x 1,000 x 5,328 370 -> 264 us, 3,000 x 300
+// x 16,384 1,010 -> 750 us; at 4,000 x 2,000 x 16,384, 512 tiles, 1,500 -> 1,590).
 template <int K>
 void launch_split_topk(const float *S, int64_t lds, int64_t N_o, const float *D, int64_t ldd,
                        int64_t N_i, int n_pix, const double *s2, const double *alpha, int tile,
@@ -1411,19 +1427,20 @@ void launch_split_topk(const float *S, int64_t lds, int64_t N_o, const float *D,
 {
     const EdgePlan p = edge_plan(N_o, N_i);
     const int n_key = (int)mtip::ceil_div(N_o, tile);
-    const dim3 grid((unsigned)(p.nwa * p.nwb + p.n_thin));
-    if (tile == BM2) {
-        hipLaunchKernelGGL((k_gemm_split<4, 4, K, false>), grid, dim3(512), 0, st, S, lds, N_o, D,
-                           ldd, N_i, n_pix, s2, alpha, p.nta, p.ntb, p.nwa, p.nwb, n_key, part);
-    } else if (p.nta * p.ntb >= 192 && (int64_t)BM2 * std::max(lds, ldd) * 4 < ((int64_t)1 << 31)) {
-        hipLaunchKernelGGL((k_gemm_split<4, 4, K, true>), grid, dim3(512), 0, st, S, lds, N_o, D,
-                           ldd, N_i, n_pix, s2, alpha, p.nta, p.ntb, p.nwa, p.nwb, n_key, part);
-    } else {
-        const int nta = (int)mtip::ceil_div(N_o, BM), ntb = (int)mtip::ceil_div(N_i, BN);
-        hipLaunchKernelGGL((k_gemm_split<2, 2, K, false>), dim3((unsigned)(nta * ntb)), dim3(256), 0,
-                           st, S, lds, N_o, D, ldd, N_i, n_pix, s2, alpha, nta, ntb, nta, ntb,
-                           n_key, part);
-    }
+    const int nta = (int)mtip::ceil_div(N_o, BM), ntb = (int)mtip::ceil_div(N_i, BN);
+#define MTIP_SPLIT(NI, WM, WN, HALVES, GRID, TA, TB, WA, WB)                                     \
+    hipLaunchKernelGGL((k_gemm_split<NI, WM, WN, K, HALVES>), dim3((unsigned)(GRID)),           \
+                       dim3(64 * WM * WN), 0, st, S, lds, N_o, D, ldd, N_i, n_pix, s2, alpha, TA, \
+                       TB, WA, WB, n_key, part)
+    if (tile == BM2)
+        MTIP_SPLIT(4, 2, 4, false, p.nwa * p.nwb + p.n_thin, p.nta, p.ntb, p.nwa, p.nwb);
+    else if (p.nta * p.ntb >= 192 && (int64_t)BM2 * std::max(lds, ldd) * 4 < ((int64_t)1 << 31))
+        MTIP_SPLIT(4, 2, 4, true, p.nwa * p.nwb + p.n_thin, p.nta, p.ntb, p.nwa, p.nwb);
+    else if (nta * ntb <= 256)
+        MTIP_SPLIT(1, 4, 2, false, nta * ntb, nta, ntb, nta, ntb);
+    else
+        MTIP_SPLIT(2, 2, 2, false, nta * ntb, nta, ntb, nta, ntb);
+#undef MTIP_SPLIT
 }
 
 template <int PREC, int K>

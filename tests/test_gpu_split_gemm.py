@@ -25,10 +25,10 @@ def _topk(S, D, K, tile, dev):
     return idx.cpu().numpy(), val.double().cpu().numpy()
 
 
-# small tiles; 13 x 16 tiles of 256 with a thin last row and column (its keys in
+# 128-row tiles of eight waves, of four (289 tiles); 13 x 16 tiles of 256 with a thin last row and column (its keys in
 # 128-row tiles, an odd number of them) and without; one pixel stage, odd stages
 @pytest.mark.parametrize("N_o,N_i,N_p,K", [(1, 1, 16, 1), (127, 129, 48, 8), (129, 300, 208, 4),
-                                           (3092, 3873, 16, 4), (3201, 3850, 80, 2),
+                                           (2100, 2050, 32, 8), (3092, 3873, 16, 4), (3201, 3850, 80, 2),
                                            (3328, 4096, 48, 1)])
 @pytest.mark.parametrize("tile", [128, 256])
 def test_split_topk_against_fp64(dev, N_o, N_i, N_p, K, tile):
