@@ -590,6 +590,11 @@ __global__ __launch_bounds__(512) void k_gemm_big(const uint8_t *__restrict__ A,
 // of 16 pixels, double-buffered: a staged row is 3 x 32 bytes and 16 more that
 // spread 16 rows over the banks.
 constexpr int kSplitK = 16;
+// Rows this short (the hierarchy's nearest-quaternion searches have 4 values in 64)
+// keep the FP32 instructions: grids have many equally near neighbours, which their
+// sums must tell apart as before, and the time is the top-K's (20,000 x 100,000 x
+// 64, 4 best: 5.3 ms, 3.9 with the split, 0.3 of it products).
+constexpr int kPlainPix = 64;
 constexpr int kSplitRow = 3 * 2 * kSplitK + 16;
 
 typedef float floatx2 __attribute__((ext_vector_type(2)));
@@ -673,7 +678,10 @@ __global__ __launch_bounds__(64 * WM * WN) void k_gemm_split(
         of_a[i] = (wave * 64 + NT * i) >> 1 < TM;
         v_st[i] = ((of_a[i] ? row : row - TM) * (int)(of_a[i] ? lda : ldb) + 8 * h_st) * 4;
     }
-    const int n_stages = (n_pix + kSplitK - 1) / kSplitK;     // loads past it read zeros
+    // loads past the last stage read zeros; rows of kPlainPix or fewer are left to
+    // the FP32 instructions below
+    const bool plain = n_pix <= kPlainPix;
+    const int n_stages = plain ? 0 : (n_pix + kSplitK - 1) / kSplitK;
     u32x4 ra[kHalves][2];
     auto load_stage = [&](int st) __attribute__((always_inline)) {
         const int ks = st * (kSplitK * 4);
@@ -787,7 +795,7 @@ __global__ __launch_bounds__(64 * WM * WN) void k_gemm_split(
         for (int j = 0; j < 2; ++j)
 #pragma unroll
             for (int v = 0; v < 16; ++v) fine &= fabsf(acc[i][j][v]) <= 3.402823466e38f;
-    if (__syncthreads_or(!fine)) {
+    if (__syncthreads_or(!fine || plain)) {
         clear();
         constexpr int PK = 32;      // pixels a stage
         for (int k0 = 0; k0 < n_pix; k0 += PK) {

@@ -27,9 +27,10 @@ def _topk(S, D, K, tile, dev):
 
 # 128-row tiles of eight waves, of four (289 tiles); 13 x 16 tiles of 256 with a thin last row and column (its keys in
 # 128-row tiles, an odd number of them) and without; one pixel stage, odd stages
-@pytest.mark.parametrize("N_o,N_i,N_p,K", [(1, 1, 16, 1), (127, 129, 48, 8), (129, 300, 208, 4),
-                                           (2100, 2050, 32, 8), (3092, 3873, 16, 4), (3201, 3850, 80, 2),
-                                           (3328, 4096, 48, 1)])
+@pytest.mark.parametrize("N_o,N_i,N_p,K", [(1, 1, 80, 1), (127, 129, 112, 8), (129, 300, 208, 4),
+                                           (200, 300, 64, 4), (2100, 2050, 96, 8),
+                                           (3092, 3873, 80, 4), (3201, 3850, 96, 2),
+                                           (3328, 4096, 112, 1)])
 @pytest.mark.parametrize("tile", [128, 256])
 def test_split_topk_against_fp64(dev, N_o, N_i, N_p, K, tile):
     print(f"case: split FP32 top-{K} {(N_o, N_i, N_p)} tile {tile}", flush=True)
@@ -56,7 +57,7 @@ def test_split_topk_against_fp64(dev, N_o, N_i, N_p, K, tile):
     assert (got <= best + 2 * tol.max(1, keepdims=True)).all()
 
 
-@pytest.mark.parametrize("shape", [(300, 200, 64), (3100, 3900, 32)])
+@pytest.mark.parametrize("shape", [(300, 200, 96), (3100, 3900, 80)])
 def test_split_topk_keeps_infinities(dev, shape):
     N_o, N_i, N_p = shape
     print(f"case: split FP32 top-K with infinities {shape}", flush=True)
