@@ -52,47 +52,88 @@ __global__ void k_count(const int32_t *__restrict__ win, int64_t win_stride, int
         atomicAdd(bad, (int)__popcll(m));
 }
 
-// One workgroup: exclusive scans of the group sizes (image offsets) and of
-// the per-group task counts; cursor = image offsets (for the scatter);
-// n_tasks[0] = number of tasks.
-__global__ __launch_bounds__(1024) void k_scan(const int32_t *__restrict__ counts, int64_t n_groups,
-                                               int32_t *__restrict__ img_off,
-                                               int32_t *__restrict__ cursor,
-                                               int32_t *__restrict__ task_off,
-                                               int32_t *__restrict__ n_tasks)
+// Exclusive scans of the group sizes (entry offsets) and of the per-group task
+// counts.  A workgroup takes kScanPer groups, in two passes over them: its sums,
+// then (k_scan_apply, after every workgroup's sums are there) the offsets from the
+// sums of the workgroups before it, which each adds up for itself (100,000 groups
+// are 98 workgroups).  One workgroup over everything took 100 us a call for
+// 100,000 groups; these two launches take 10.
+constexpr int kScanPer = 1024;
+
+__device__ __forceinline__ int2 block_sum_int2(int a, int b, int2 *red)
 {
-    __shared__ int32_t s_a[1024], s_b[1024];
-    const int tid = threadIdx.x;
-    const int64_t per = (n_groups + 1023) / 1024;
-    const int64_t g0 = tid * per, g1 = min(n_groups, g0 + per);
-    int32_t a = 0, b = 0;
-    for (int64_t g = g0; g < g1; ++g) {
-        a += counts[g];
-        b += (counts[g] + kTaskImages - 1) / kTaskImages;
+    for (int m = 32; m >= 1; m >>= 1) {
+        a += __shfl_xor(a, m, 64);
+        b += __shfl_xor(b, m, 64);
     }
-    s_a[tid] = a;
-    s_b[tid] = b;
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = make_int2(a, b);
     __syncthreads();
-    // Hillis-Steele inclusive scan over the 1024 partial sums
-    for (int d = 1; d < 1024; d <<= 1) {
-        int32_t va = tid >= d ? s_a[tid - d] : 0, vb = tid >= d ? s_b[tid - d] : 0;
-        __syncthreads();
-        s_a[tid] += va;
-        s_b[tid] += vb;
-        __syncthreads();
+    int2 t = make_int2(0, 0);
+    for (int w = 0; w < (int)(blockDim.x >> 6); ++w) {
+        t.x += red[w].x;
+        t.y += red[w].y;
     }
-    int32_t ra = s_a[tid] - a, rb = s_b[tid] - b;     // exclusive
-    for (int64_t g = g0; g < g1; ++g) {
+    __syncthreads();
+    return t;
+}
+
+__global__ __launch_bounds__(kScanPer) void k_scan_sums(const int32_t *__restrict__ counts,
+                                                        int64_t n_groups, int2 *__restrict__ sums)
+{
+    __shared__ int2 red[kScanPer / 64];
+    const int64_t g = (int64_t)blockIdx.x * kScanPer + threadIdx.x;
+    const int c = g < n_groups ? counts[g] : 0;
+    const int2 t = block_sum_int2(c, (c + kTaskImages - 1) / kTaskImages, red);
+    if (threadIdx.x == 0) sums[blockIdx.x] = t;
+}
+
+// img_off, task_off: the scans; cursor = entry offsets (for the scatter);
+// n_tasks[0] = number of tasks.
+__global__ __launch_bounds__(kScanPer) void k_scan_apply(const int32_t *__restrict__ counts,
+                                                         int64_t n_groups,
+                                                         const int2 *__restrict__ sums,
+                                                         int32_t *__restrict__ img_off,
+                                                         int32_t *__restrict__ cursor,
+                                                         int32_t *__restrict__ task_off,
+                                                         int32_t *__restrict__ n_tasks)
+{
+    __shared__ int2 red[kScanPer / 64];
+    __shared__ int2 s_wave[kScanPer / 64];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    int a = 0, b = 0;
+    for (int k = tid; k < (int)blockIdx.x; k += kScanPer) {
+        a += sums[k].x;
+        b += sums[k].y;
+    }
+    const int2 before = block_sum_int2(a, b, red);
+    const int64_t g = (int64_t)blockIdx.x * kScanPer + tid;
+    const int c = g < n_groups ? counts[g] : 0;
+    const int ct = (c + kTaskImages - 1) / kTaskImages;
+    a = c;
+    b = ct;
+    for (int d = 1; d < 64; d <<= 1) {
+        const int ua = __shfl_up(a, d, 64), ub = __shfl_up(b, d, 64);
+        if (lane >= d) {
+            a += ua;
+            b += ub;
+        }
+    }
+    if (lane == 63) s_wave[wave] = make_int2(a, b);
+    __syncthreads();
+    int ra = before.x + a - c, rb = before.y + b - ct;     // exclusive
+    for (int w = 0; w < wave; ++w) {
+        ra += s_wave[w].x;
+        rb += s_wave[w].y;
+    }
+    if (g < n_groups) {
         img_off[g] = ra;
         cursor[g] = ra;
         task_off[g] = rb;
-        ra += counts[g];
-        rb += (counts[g] + kTaskImages - 1) / kTaskImages;
     }
-    if (tid == 1023) {
-        img_off[n_groups] = s_a[1023];
-        cursor[n_groups] = s_a[1023];     // entries left out go after the grouped ones
-        n_tasks[0] = s_b[1023];
+    if (g == n_groups - 1) {
+        img_off[n_groups] = ra + c;
+        cursor[n_groups] = ra + c;     // entries left out go after the grouped ones
+        n_tasks[0] = rb + ct;
     }
 }
 
@@ -365,18 +406,25 @@ __global__ __launch_bounds__(256) void k_group_topk(
 }
 
 // Per image: the K_out smallest distinct keys among its n_in candidate
-// (index, value) pairs (T entries x K each, index -1 = none).
+// (index, value) pairs (T entries x K each, index -1 = none).  One wave per image:
+// each lane keeps the smallest distinct keys of every 64th pair, then the wave
+// takes its minimum K_out times, every lane that holds it dropping it.  (A thread
+// per image left 12,000 images to 48 workgroups reading 512 pairs one by one: 280
+// us; a wave takes 32.)
 template <int KO>
-__global__ void k_merge_distinct(const int32_t *__restrict__ in_idx,
-                                 const float *__restrict__ in_val, int64_t N_i, int n_in,
-                                 int32_t *__restrict__ out_idx, float *__restrict__ out_val)
+__global__ __launch_bounds__(256) void k_merge_distinct(const int32_t *__restrict__ in_idx,
+                                                        const float *__restrict__ in_val,
+                                                        int64_t N_i, int n_in,
+                                                        int32_t *__restrict__ out_idx,
+                                                        float *__restrict__ out_val)
 {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int lane = threadIdx.x & 63;
+    const int64_t i = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
     if (i >= N_i) return;
     uint64_t top[KO];
 #pragma unroll
     for (int r = 0; r < KO; ++r) top[r] = KEY_NONE;
-    for (int j = 0; j < n_in; ++j) {
+    for (int j = lane; j < n_in; j += 64) {
         const int32_t id = in_idx[i * n_in + j];
         if (id < 0) continue;
         const uint64_t key = mtip::make_key(in_val[i * n_in + j], (uint32_t)id);
@@ -385,11 +433,23 @@ __global__ void k_merge_distinct(const int32_t *__restrict__ in_idx,
         for (int r = 0; r < KO; ++r) dup |= (top[r] == key);
         if (!dup) mtip::topk_insert<KO>(top, key);
     }
-#pragma unroll
+#pragma unroll 1
     for (int r = 0; r < KO; ++r) {
-        const bool ok = top[r] != KEY_NONE;
-        out_idx[i * KO + r] = ok ? (int32_t)(uint32_t)top[r] : -1;
-        out_val[i * KO + r] = ok ? mtip::ordered_to_float((uint32_t)(top[r] >> 32)) : __builtin_inff();
+        uint64_t m = top[0];
+        for (int d = 32; d >= 1; d >>= 1) {
+            const uint64_t o = mtip::shfl_xor_u64(m, d);
+            m = o < m ? o : m;
+        }
+        if (top[0] == m) {
+#pragma unroll
+            for (int e = 0; e + 1 < KO; ++e) top[e] = top[e + 1];
+            top[KO - 1] = KEY_NONE;
+        }
+        if (lane == 0) {
+            const bool ok = m != KEY_NONE;
+            out_idx[i * KO + r] = ok ? (int32_t)(uint32_t)m : -1;
+            out_val[i * KO + r] = ok ? mtip::ordered_to_float((uint32_t)(m >> 32)) : __builtin_inff();
+        }
     }
 }
 
@@ -486,8 +546,12 @@ extern "C" int mtip_group_by_winner(const int32_t *winners, int64_t win_stride, 
     if (N_e > 0)
         hipLaunchKernelGGL(k_count, dim3((unsigned)mtip::ceil_div(N_e, 256)), dim3(256), 0, st,
                            winners, win_stride, (int64_t)n_win, N_e, n_groups, w.counts, w.bad);
-    hipLaunchKernelGGL(k_scan, dim3(1), dim3(1024), 0, st, w.counts, n_groups, w.img_off,
-                       w.cursor, w.task_off, w.n_tasks);
+    // the workgroups' sums go where the tasks will be written (k_tasks runs last)
+    const unsigned n_scan = (unsigned)mtip::ceil_div(n_groups, kScanPer);
+    hipLaunchKernelGGL(k_scan_sums, dim3(n_scan), dim3(kScanPer), 0, st, w.counts, n_groups,
+                       (int2 *)w.tasks);
+    hipLaunchKernelGGL(k_scan_apply, dim3(n_scan), dim3(kScanPer), 0, st, w.counts, n_groups,
+                       (const int2 *)w.tasks, w.img_off, w.cursor, w.task_off, w.n_tasks);
     if (N_e > 0)
         hipLaunchKernelGGL(k_scatter, dim3((unsigned)mtip::ceil_div(N_e, 256)), dim3(256), 0, st,
                            winners, win_stride, (int64_t)n_win, N_e, n_groups, w.cursor, w.perm);
@@ -631,7 +695,7 @@ extern "C" int mtip_merge_distinct(const int32_t *in_idx, const float *in_val, i
     MTIP_REQUIRE(in_idx && in_val && out_idx && out_val, MTIP_ERR_ARG,
                  "mtip_merge_distinct: null pointer");
     hipStream_t st = (hipStream_t)stream;
-    const dim3 grid((unsigned)mtip::ceil_div(N_i, 256));
+    const dim3 grid((unsigned)mtip::ceil_div(N_i, 4));
     switch (K_out) {
     case 1: hipLaunchKernelGGL(k_merge_distinct<1>, grid, dim3(256), 0, st, in_idx, in_val, N_i, n_in, out_idx, out_val); break;
     case 2: hipLaunchKernelGGL(k_merge_distinct<2>, grid, dim3(256), 0, st, in_idx, in_val, N_i, n_in, out_idx, out_val); break;
