@@ -388,6 +388,16 @@ __device__ __forceinline__ void taps_pair_direct(__amdgpu_buffer_rsrc_t rsrc, in
     r1 = a1;
 }
 
+// TP = points per tile.  A trip takes 256 points, so every thread computes the
+// geometry of one point (FP64 rotation and window corner) whatever the tile; the
+// 256 / TP tiles of the trip are then staged one after the other by all four waves.
+// Bound: VALU (about 2,100 instructions per 64 points at TP = 64, three quarters of
+// them geometry, weights and staging around the taps) with the LDS 70 % active.
+// One tile per trip left three of four waves idle in the geometry at TP = 64 and
+// took three barriers a tile instead of about one and a half: M = 121, 1,024 x 16k
+// points 1,830 us, now 1,550; 10k x 12.4k points 12.4 ms, now 10.7.  TP = 256 is one
+// tile a trip either way.  More staging loads in flight, running quotients for the
+// chunk addresses and 24-bit products all spill at 168 registers and lose.
 template <int W, int TP>
 __global__ __launch_bounds__(256, 3) void k_slices_lds(GridView gv, const double *__restrict__ quats,
                                                     const double *__restrict__ q, int64_t N_p,
@@ -402,14 +412,14 @@ __global__ __launch_bounds__(256, 3) void k_slices_lds(GridView gv, const double
 {
     using PT = PairTaps<W>;
     constexpr int GP = PT::GP, NS = PT::NS, PPW = 64 / GP;
+    constexpr int NSUB = 256 / TP;                              // tiles per trip
     constexpr int PW = TP / 4;                                  // points per wave
     constexpr int STEPS = PW >= PPW ? PW / PPW : 1;
     __shared__ __align__(16) float s_box[kBoxCap];
     // per point: pair-base offset (box-local when staged, padded grid otherwise)
     // with the window parity in bit 0, or -1 for a point outside the domain
-    __shared__ int s_lb[TP];
-    __shared__ int s_pix[TP];          // output pixel, -1 for an empty slot
-    __shared__ float s_t[3][TP];       // fractional window offsets
+    __shared__ int s_lb[256];
+    __shared__ float s_t[3][256];      // fractional window offsets
     __shared__ int s_red_i[4][6];
     __shared__ double s_red[8];
 
@@ -438,13 +448,11 @@ __global__ __launch_bounds__(256, 3) void k_slices_lds(GridView gv, const double
     uint16_t *brow = out_bf16 ? out_bf16 + o * ld_out : nullptr;
     double sum = 0.0, sumsq = 0.0;
     int nbad = 0;
-    const int64_t n_slots = order ? n_order : mtip::ceil_div(N_p, TP) * TP;
-    const bool has_pt = tid < TP;      // threads holding a point of the tile
+    const int64_t n_slots = order ? n_order : N_p;
 
-    // pixel index and q-vector of this thread's point, prefetched one tile ahead
-    // (and the pixel index two tiles ahead) so their latency hides behind taps
+    // pixel index and q-vector of this thread's point, prefetched one trip ahead
+    // (and the pixel index two trips ahead) so their latency hides behind taps
     auto pixel_at = [&](int64_t k) -> int {
-        if (!has_pt) return -1;
         if (order) return (k < n_order) ? order[k] : -1;
         return (k < N_p) ? (int)k : -1;
     };
@@ -456,9 +464,9 @@ __global__ __launch_bounds__(256, 3) void k_slices_lds(GridView gv, const double
         qy_n = q[N_p + pp];
         qz_n = q[2 * N_p + pp];
     }
-    int pix_nn = pixel_at(TP + tid);
+    int pix_nn = pixel_at(256 + tid);
 
-    for (int64_t tb = 0; tb < n_slots; tb += TP) {
+    for (int64_t tb = 0; tb < n_slots; tb += 256) {
         // ---- geometry of this thread's point
         const int pix = pix_n;
         const double x = qx_n, y = qy_n, z = qz_n;
@@ -469,7 +477,7 @@ __global__ __launch_bounds__(256, 3) void k_slices_lds(GridView gv, const double
             qy_n = q[N_p + pp];
             qz_n = q[2 * N_p + pp];
         }
-        pix_nn = pixel_at(tb + 2 * TP + tid);
+        pix_nn = pixel_at(tb + 512 + tid);
         bool ok = false;
         int ijk[3] = {0, 0, 0};
         float t[3] = {0.f, 0.f, 0.f};
@@ -479,7 +487,7 @@ __global__ __launch_bounds__(256, 3) void k_slices_lds(GridView gv, const double
             double X2 = (s_ri[6] * x + s_ri[7] * y + s_ri[8] * z) * gscale;
             ok = point_corner<W>(gv, X0, X1, X2, ijk, t);
         }
-        // ---- box of the tile's windows (block min / max)
+        // ---- box of each wave's windows (min / max)
         {
             int v[6] = {ok ? ijk[0] : 0x7fffffff, ok ? ijk[1] : 0x7fffffff, ok ? ijk[2] : 0x7fffffff,
                         ok ? -ijk[0] : 0x7fffffff, ok ? -ijk[1] : 0x7fffffff, ok ? -ijk[2] : 0x7fffffff};
@@ -489,141 +497,154 @@ __global__ __launch_bounds__(256, 3) void k_slices_lds(GridView gv, const double
 #pragma unroll
                 for (int e = 0; e < 6; ++e) s_red_i[wave][e] = v[e];
         }
+        s_t[0][tid] = t[0];
+        s_t[1][tid] = t[1];
+        s_t[2][tid] = t[2];
         __syncthreads();
-        int lo[3], hi[3];
-#pragma unroll
-        for (int e = 0; e < 3; ++e) {
-            lo[e] = min(min(s_red_i[0][e], s_red_i[1][e]), min(s_red_i[2][e], s_red_i[3][e]));
-            hi[e] = -min(min(s_red_i[0][e + 3], s_red_i[1][e + 3]),
-                         min(s_red_i[2][e + 3], s_red_i[3][e + 3]));
-        }
-        const bool any = lo[0] != 0x7fffffff;
-        const int lz = lo[2] & ~1;      // even, so every pair base is 8-byte aligned
-        const int bx = any ? hi[0] - lo[0] + W : 0, by = any ? hi[1] - lo[1] + W : 0;
-        const int bz = any ? hi[2] - lz + 2 * GP : 0;
-        const int S = pair_stride(bz);
-        // plane stride: by * S raised to 10 mod 32 floats when the box still
-        // fits.  A quarter-wave serves a 2 x 2 pixel group whose window
-        // corners differ by about one cell per axis; with 32 banks, neighbours
-        // one plane apart then read other banks.  Measured over residues at
-        // M = 81, 10k x 16k: 8.75 ms at 10 mod 32 against 8.98 ms unpadded (a
-        // quarter-wave bank model ranks the residues alike; 0 and 6 are worst)
-        int plane = by * S;
-        {
-            const int padded = plane + ((10 - plane) & 31);
-            if (bx * padded <= kBoxCap) plane = padded;
-        }
-        const bool staged = any && S > 0 && bx * plane <= kBoxCap;
-        // this point's pair base (box-local when staged, padded grid otherwise)
-        int lb = -1;
-        if (ok) {
-            const int zb = ijk[2] & ~1;
-            lb = staged ? (ijk[0] - lo[0]) * plane + (ijk[1] - lo[1]) * S + (zb - lz)
-                        : (ijk[0] * np + ijk[1]) * np + zb;
-            lb |= ijk[2] & 1;
-        }
-
-        if (has_pt) {
-            s_lb[tid] = lb;
-            s_pix[tid] = pix;
-            s_t[0][tid] = t[0];
-            s_t[1][tid] = t[1];
-            s_t[2][tid] = t[2];
-        }
-        // ---- the box
-        if (staged) {
-            // the box as nrows * q4 chunks of 16 bytes, chunk k = row k / q4,
-            // quarter k % q4: every thread's loads go in flight at once (at most
-            // kStageChunks each, enough for any box within kBoxCap), then the
-            // 8-byte LDS stores (pairs at or past S dropped)
-            const int q4 = (bz + 3) >> 2;
-            const int nchunk = bx * by * q4;
-            const float inv_q4 = 1.0f / (float)q4, inv_by = 1.0f / (float)by;
-            auto stage = [&](int u0, auto nb) __attribute__((always_inline)) {
-                constexpr int NB = decltype(nb)::value;
-                uint4v v[NB];
-#pragma unroll
-                for (int u = 0; u < NB; ++u) {
-                    const int k = (u0 + u) * 256 + tid;
-                    // k / q4 and r / by for k < 2^16: the float estimates are
-                    // within half a unit of the integer quotient
-                    const int r = (int)(((float)k + 0.5f) * inv_q4), zq = k - r * q4;
-                    const int xr = (int)(((float)r + 0.5f) * inv_by), yr = r - xr * by;
-                    const int gidx =
-                        k < nchunk ? ((lo[0] + xr) * np + (lo[1] + yr)) * np + lz + 4 * zq : 0;
-                    v[u] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, gidx * 4, 0, 0);
-                }
-#pragma unroll
-                for (int u = 0; u < NB; ++u) {
-                    const int k = (u0 + u) * 256 + tid;
-                    if (k < nchunk) {
-                        const int r = (int)(((float)k + 0.5f) * inv_q4), z4 = 4 * (k - r * q4);
-                        const int xr = (int)(((float)r + 0.5f) * inv_by), yr = r - xr * by;
-                        float2 *d2 = reinterpret_cast<float2 *>(s_box + xr * plane + yr * S + z4);
-                        d2[0] = make_float2(__uint_as_float(v[u][0]), __uint_as_float(v[u][1]));
-                        if (z4 + 2 < S)
-                            d2[1] = make_float2(__uint_as_float(v[u][2]), __uint_as_float(v[u][3]));
-                    }
-                }
-            };
-            stage(0, std::integral_constant<int, kStageChunks>{});
-            for (int u0 = kStageChunks; u0 * 256 < nchunk; u0 += 4)
-                stage(u0, std::integral_constant<int, 4>{});
-        }
-        __syncthreads();
-        // ---- taps: each wave its PW points, PPW per step
+        // ---- the tiles of this trip, one after the other: the four waves stage a
+        // tile's box and share its points.  Boxes lie at the two ends of s_box in
+        // turn, so a box that leaves room for the one before it is staged without
+        // waiting for that one's readers
+        int room = kBoxCap;       // not taken by the tile before
 #pragma unroll 1
-        for (int it = 0; it < STEPS; ++it) {
-            const bool slot_ok = PW >= PPW || g < PW;
-            const int pl = slot_ok ? wave * PW + it * PPW + g : 0;
-            const int lv = s_lb[pl];
-            const float tx = s_t[0][pl], ty = s_t[1][pl], tz = s_t[2][pl];
-            const int sh = lv & 1;
-            const int base = lv >= 0 ? (lv & ~1) + 2 * c : 0;
-            float own_a[NS], own_b[NS];
+        for (int sub = 0; sub < NSUB; ++sub) {
+            int lo[3], hi[3];
 #pragma unroll
-            for (int s = 0; s < NS; ++s) {
-                own_a[s] = es_phi((float)(c + GP * s) - tx, gv.beta_l2e, gv.c2);
-                own_b[s] = es_phi((float)(c + GP * s) - ty, gv.beta_l2e, gv.c2);
-            }
-            float wa[W], wb[W];
-            gather_weights<GP, W>(own_a, wa, lane);
-            gather_weights<GP, W>(own_b, wb, lane);
-            // elements 2c - sh and 2c + 1 - sh of the window (zero weight outside it)
-            const float k0 = (float)(2 * c - sh);
-            const float wc0 = es_phi(k0 - tz, gv.beta_l2e, gv.c2);
-            const float wc1 = es_phi(k0 + 1.0f - tz, gv.beta_l2e, gv.c2);
-            float r0 = 0.f, r1 = 0.f;
-            if (staged) {
-                switch (S) {
-#define MTIP_TAPS_CASE(SS) case SS: taps_pair_lds<W, SS>(s_box, base, plane, wa, wb, r0, r1); break;
-                    MTIP_PAIR_STRIDES(MTIP_TAPS_CASE)
-#undef MTIP_TAPS_CASE
-                default: break;
+            for (int e = 0; e < 3; ++e) {
+                lo[e] = 0x7fffffff;
+                hi[e] = 0x7fffffff;
+#pragma unroll
+                for (int w = 0; w < 4 / NSUB; ++w) {
+                    lo[e] = min(lo[e], s_red_i[sub * (4 / NSUB) + w][e]);
+                    hi[e] = min(hi[e], s_red_i[sub * (4 / NSUB) + w][e + 3]);
                 }
-            } else {
-                taps_pair_direct<W>(rsrc, np, base * 4, wa, wb, r0, r1);
+                hi[e] = -hi[e];
             }
-            const float r = group_sum<GP>(fmaf(wc0, r0, wc1 * r1));
-            // the slot's value replaces its x offset (read above, by this wave only)
-            if (c == 0 && slot_ok) s_t[0][pl] = r;
+            const bool any = lo[0] != 0x7fffffff;
+            const int lz = lo[2] & ~1;      // even, so every pair base is 8-byte aligned
+            const int bx = any ? hi[0] - lo[0] + W : 0, by = any ? hi[1] - lo[1] + W : 0;
+            const int bz = any ? hi[2] - lz + 2 * GP : 0;
+            const int S = pair_stride(bz);
+            // plane stride: by * S raised to 10 mod 32 floats when the box still
+            // fits.  A quarter-wave serves a 2 x 2 pixel group whose window
+            // corners differ by about one cell per axis; with 32 banks, neighbours
+            // one plane apart then read other banks.  Measured over residues at
+            // M = 81, 10k x 16k: 8.75 ms at 10 mod 32 against 8.98 ms unpadded (a
+            // quarter-wave bank model ranks the residues alike; 0 and 6 are worst)
+            int plane = by * S;
+            {
+                const int padded = plane + ((10 - plane) & 31);
+                if (bx * padded <= kBoxCap) plane = padded;
+            }
+            const bool staged = any && S > 0 && bx * plane <= kBoxCap;
+            float *const box = s_box + (NSUB > 1 && (sub & 1) && staged ? kBoxCap - bx * plane : 0);
+            // this point's pair base (box-local when staged, padded grid otherwise)
+            if (NSUB == 1 || tid / TP == sub) {
+                int lb = -1;
+                if (ok) {
+                    const int zb = ijk[2] & ~1;
+                    lb = staged ? (ijk[0] - lo[0]) * plane + (ijk[1] - lo[1]) * S + (zb - lz)
+                                : (ijk[0] * np + ijk[1]) * np + zb;
+                    lb |= ijk[2] & 1;
+                }
+                s_lb[tid] = lb;
+            }
+            // ---- the box
+            if (staged) {
+                if (NSUB > 1) {
+                    if (bx * plane > room) __syncthreads();
+                    room = kBoxCap - bx * plane;
+                }
+                // the box as nrows * q4 chunks of 16 bytes, chunk k = row k / q4,
+                // quarter k % q4: every thread's loads go in flight at once (at most
+                // kStageChunks each, enough for any box within kBoxCap), then the
+                // 8-byte LDS stores (pairs at or past S dropped)
+                const int q4 = (bz + 3) >> 2;
+                const int nchunk = bx * by * q4;
+                const float inv_q4 = 1.0f / (float)q4, inv_by = 1.0f / (float)by;
+                auto stage = [&](int u0, auto nb) __attribute__((always_inline)) {
+                    constexpr int NB = decltype(nb)::value;
+                    uint4v v[NB];
+#pragma unroll
+                    for (int u = 0; u < NB; ++u) {
+                        const int k = (u0 + u) * 256 + tid;
+                        // k / q4 and r / by for k < 2^16: the float estimates are
+                        // within half a unit of the integer quotient
+                        const int r = (int)(((float)k + 0.5f) * inv_q4), zq = k - r * q4;
+                        const int xr = (int)(((float)r + 0.5f) * inv_by), yr = r - xr * by;
+                        const int gidx =
+                            k < nchunk ? ((lo[0] + xr) * np + (lo[1] + yr)) * np + lz + 4 * zq : 0;
+                        v[u] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, gidx * 4, 0, 0);
+                    }
+#pragma unroll
+                    for (int u = 0; u < NB; ++u) {
+                        const int k = (u0 + u) * 256 + tid;
+                        if (k < nchunk) {
+                            const int r = (int)(((float)k + 0.5f) * inv_q4), z4 = 4 * (k - r * q4);
+                            const int xr = (int)(((float)r + 0.5f) * inv_by), yr = r - xr * by;
+                            float2 *d2 = reinterpret_cast<float2 *>(box + xr * plane + yr * S + z4);
+                            d2[0] = make_float2(__uint_as_float(v[u][0]), __uint_as_float(v[u][1]));
+                            if (z4 + 2 < S)
+                                d2[1] = make_float2(__uint_as_float(v[u][2]), __uint_as_float(v[u][3]));
+                        }
+                    }
+                };
+                stage(0, std::integral_constant<int, kStageChunks>{});
+                for (int u0 = kStageChunks; u0 * 256 < nchunk; u0 += 4)
+                    stage(u0, std::integral_constant<int, 4>{});
+            }
+            __syncthreads();
+            // ---- taps: each wave its PW points, PPW per step
+#pragma unroll 1
+            for (int it = 0; it < STEPS; ++it) {
+                const bool slot_ok = PW >= PPW || g < PW;
+                const int pl = sub * TP + (slot_ok ? wave * PW + it * PPW + g : 0);
+                const int lv = s_lb[pl];
+                const float tx = s_t[0][pl], ty = s_t[1][pl], tz = s_t[2][pl];
+                const int sh = lv & 1;
+                const int base = lv >= 0 ? (lv & ~1) + 2 * c : 0;
+                float own_a[NS], own_b[NS];
+#pragma unroll
+                for (int s = 0; s < NS; ++s) {
+                    own_a[s] = es_phi((float)(c + GP * s) - tx, gv.beta_l2e, gv.c2);
+                    own_b[s] = es_phi((float)(c + GP * s) - ty, gv.beta_l2e, gv.c2);
+                }
+                float wa[W], wb[W];
+                gather_weights<GP, W>(own_a, wa, lane);
+                gather_weights<GP, W>(own_b, wb, lane);
+                // elements 2c - sh and 2c + 1 - sh of the window (zero weight outside it)
+                const float k0 = (float)(2 * c - sh);
+                const float wc0 = es_phi(k0 - tz, gv.beta_l2e, gv.c2);
+                const float wc1 = es_phi(k0 + 1.0f - tz, gv.beta_l2e, gv.c2);
+                float r0 = 0.f, r1 = 0.f;
+                if (staged) {
+                    switch (S) {
+#define MTIP_TAPS_CASE(SS) case SS: taps_pair_lds<W, SS>(box, base, plane, wa, wb, r0, r1); break;
+                        MTIP_PAIR_STRIDES(MTIP_TAPS_CASE)
+#undef MTIP_TAPS_CASE
+                    default: break;
+                    }
+                } else {
+                    taps_pair_direct<W>(rsrc, np, base * 4, wa, wb, r0, r1);
+                }
+                const float r = group_sum<GP>(fmaf(wc0, r0, wc1 * r1));
+                // the slot's value replaces its x offset (read above, by this wave only)
+                if (c == 0 && slot_ok) s_t[0][pl] = r;
+            }
         }
         // ---- outputs: each thread its own slot (written by its own wave when TP = 256)
         if constexpr (TP == 256) wave_sync();
         else __syncthreads();
-        if (has_pt) {
-            const int pix_o = s_pix[tid];
-            if (pix_o >= 0) {
-                float v = s_t[0][tid];
-                if (s_lb[tid] < 0) {
-                    v = __builtin_nanf("");
-                    ++nbad;
-                }
-                orow[pix_o] = v;
-                if (brow) brow[pix_o] = f32_to_bf16_rne(v);
-                sum += (double)v;
-                sumsq += (double)v * (double)v;
+        if (pix >= 0) {
+            float v = s_t[0][tid];
+            if (s_lb[tid] < 0) {
+                v = __builtin_nanf("");
+                ++nbad;
             }
+            orow[pix] = v;
+            if (brow) brow[pix] = f32_to_bf16_rne(v);
+            sum += (double)v;
+            sumsq += (double)v * (double)v;
         }
         __syncthreads();
     }
