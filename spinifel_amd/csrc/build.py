@@ -13,7 +13,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 PKG = os.path.dirname(HERE)
 ROOT = os.path.dirname(PKG)
 OUT = os.path.join(PKG, "libmtip.so")
-SOURCES = ["common.hip", "nufft.hip", "adjoint.hip", "match.hip", "hier.hip", "phasing.hip", "prep.hip", "merge.hip", "static_match.hip"]
+SOURCES = ["common.hip", "nufft.hip", "dft.hip", "adjoint.hip", "match.hip", "hier.hip", "phasing.hip", "prep.hip", "merge.hip", "static_match.hip"]
 ARCH = "gfx950"
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
@@ -52,8 +52,7 @@ def build(verbose=False, jobs=None):
     if failed:
         raise RuntimeError(f"hipcc failed for {failed}")
     tmp = OUT + ".tmp"
-    cmd = [HIPCC, "-shared", f"--offload-arch={ARCH}", "-fPIC", *objs, "-L/opt/rocm/lib",
-           "-lhipfft", "-Wl,-rpath,/opt/rocm/lib", "-o", tmp]
+    cmd = [HIPCC, "-shared", f"--offload-arch={ARCH}", "-fPIC", *objs, "-o", tmp]
     subprocess.run(cmd, check=True)
     os.replace(tmp, OUT)
     return OUT

@@ -6,14 +6,12 @@
 //   b_l    = sum_k g_k exp(-2 pi i k . l / n),  g_k = sym(a)_k / prod phihat(k_d)
 //   Re c_j = sum_l b_l prod_d phi(X_jd - l_d),  X = x n / (2 pi)
 // sym(a)_k = (a(k) + a(-k)) / 2 makes b real (the reference keeps only the
-// real part of the transform); b comes from one FP64 hipFFT transform of the
-// n^3 grid, and the fine grid is a real float32 array of
+// real part of the transform); b comes from one FP64 transform (dft.hip), and
+// the fine grid is a real float32 array of
 // (n + 2 pad)^3 values, indices l in [-n/2 - pad, n/2 + pad), evaluated
 // directly at the padded indices so no wrap is needed while interpolating.
 #include <math.h>
 #include <vector>
-
-#include <hipfft/hipfft.h>
 
 #include "nufft_shared.h"
 
@@ -84,46 +82,6 @@ __global__ void k_twiddle(double2 *tw, int n)
         sincospi(2.0 * (double)m / (double)n, &s, &c);
         tw[m] = make_double2(c, -s);
     }
-}
-
-// Fine grid by FFT: G holds g_k = sym(a)_k / prod phihat(k_d) at index
-// k mod n (zero elsewhere), one thread per G entry so no clearing pass is
-// needed; hipFFT's forward Z2Z gives b_l = sum_k g_k exp(-2 pi i k . l / n),
-// real because g is real and even; k_pad_grid writes b at the padded indices
-// (periodic in l) as float32.
-__global__ __launch_bounds__(256) void k_scatter_model(const float *__restrict__ ac,
-                                                       const double *__restrict__ dinv,
-                                                       double2 *__restrict__ G, int M, int h,
-                                                       int n)
-{
-    const int64_t n3 = (int64_t)n * n * n;
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n3) return;
-    const int i3 = (int)(i % n), i2 = (int)((i / n) % n), i1 = (int)(i / ((int64_t)n * n));
-    const int k1 = i1 <= n / 2 ? i1 : i1 - n, k2 = i2 <= n / 2 ? i2 : i2 - n,
-              k3 = i3 <= n / 2 ? i3 : i3 - n;
-    double v = 0.0;
-    if (abs(k1) <= h && abs(k2) <= h && abs(k3) <= h) {
-        const int lo = -(M / 2), hi = (M - 1) / 2;
-        double s = 0.0;
-        if (k1 >= lo && k1 <= hi && k2 >= lo && k2 <= hi && k3 >= lo && k3 <= hi)
-            s += ac[((int64_t)(k1 + M / 2) * M + (k2 + M / 2)) * M + (k3 + M / 2)];
-        if (-k1 >= lo && -k1 <= hi && -k2 >= lo && -k2 <= hi && -k3 >= lo && -k3 <= hi)
-            s += ac[((int64_t)(-k1 + M / 2) * M + (-k2 + M / 2)) * M + (-k3 + M / 2)];
-        v = 0.5 * s * dinv[k1 + h] * dinv[k2 + h] * dinv[k3 + h];
-    }
-    G[i] = make_double2(v, 0.0);
-}
-
-__global__ __launch_bounds__(256) void k_pad_grid(const double2 *__restrict__ G,
-                                                  float *__restrict__ grid, int n, int np, int off)
-{
-    const int64_t np3 = (int64_t)np * np * np;
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= np3) return;
-    const int p3 = (int)(i % np), p2 = (int)((i / np) % np), p1 = (int)(i / ((int64_t)np * np));
-    auto wrap = [n, off](int p) { return ((p - off) % n + n) % n; };
-    grid[i] = (float)G[((int64_t)wrap(p1) * n + wrap(p2)) * n + wrap(p3)].x;
 }
 
 // ------------------------------------------------------------ interpolation
@@ -773,7 +731,6 @@ extern "C" int mtip_plan_destroy(mtip_plan *p)
     (void)hipFree(p->dinv);
     (void)hipFree(p->tw);
     (void)hipFree(p->G);
-    if (p->fft) (void)hipfftDestroy((hipfftHandle)p->fft);
     (void)hipFree(p->acc);
     (void)hipFree(p->a1);
     (void)hipFree(p->a2);
@@ -798,37 +755,8 @@ extern "C" int mtip_plan_set_model(mtip_plan *p, const float *ac, void *stream)
     DeviceGuard dg(p->device);
     MTIP_REQUIRE(dg.ok, MTIP_ERR_HIP, "mtip_plan_set_model: cannot select device");
     hipStream_t st = (hipStream_t)stream;
-    const int64_t n3 = (int64_t)p->n * p->n * p->n;
-    const int64_t np3 = (int64_t)p->np * p->np * p->np;
-    if (!p->G) {
-        // first model on this plan: the FFT buffer and plan (plans used only
-        // for the adjoint never need them)
-        hipError_t e = hipMalloc(&p->G, (size_t)n3 * sizeof(double2));
-        if (e != hipSuccess) {
-            p->G = nullptr;
-            return mtip::fail(e == hipErrorOutOfMemory ? MTIP_ERR_NOMEM : MTIP_ERR_HIP,
-                              std::string("mtip_plan_set_model: ") + hipGetErrorString(e));
-        }
-        hipfftHandle fh = nullptr;
-        if (hipfftPlan3d(&fh, p->n, p->n, p->n, HIPFFT_Z2Z) != HIPFFT_SUCCESS) {
-            (void)hipFree(p->G);
-            p->G = nullptr;
-            return mtip::fail(MTIP_ERR_HIP, "mtip_plan_set_model: hipfftPlan3d failed");
-        }
-        p->fft = fh;
-    }
-    hipLaunchKernelGGL(k_scatter_model, dim3((unsigned)mtip::ceil_div(n3, 256)), dim3(256), 0, st,
-                       ac, p->dinv, p->G, p->M, p->h, p->n);
-    MTIP_HIP_CHECK(hipGetLastError());
-    hipfftHandle fh = (hipfftHandle)p->fft;
-    MTIP_REQUIRE(hipfftSetStream(fh, st) == HIPFFT_SUCCESS, MTIP_ERR_HIP,
-                 "mtip_plan_set_model: hipfftSetStream failed");
-    MTIP_REQUIRE(hipfftExecZ2Z(fh, (hipfftDoubleComplex *)p->G, (hipfftDoubleComplex *)p->G,
-                               HIPFFT_FORWARD) == HIPFFT_SUCCESS,
-                 MTIP_ERR_HIP, "mtip_plan_set_model: hipfftExecZ2Z failed");
-    hipLaunchKernelGGL(k_pad_grid, dim3((unsigned)mtip::ceil_div(np3, 256)), dim3(256), 0, st,
-                       p->G, p->grid, p->n, p->np, p->off);
-    MTIP_HIP_CHECK(hipGetLastError());
+    const int rc = mtip::grid_from_model(p, ac, st);
+    if (rc != MTIP_OK) return rc;
     p->loaded = true;
     return MTIP_OK;
 }

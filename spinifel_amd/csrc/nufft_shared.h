@@ -16,8 +16,7 @@ struct mtip_plan {
     float *grid = nullptr;        // (np)^3 real fine grid
     double *dinv = nullptr;       // K: 1 / phihat(k)
     double2 *tw = nullptr;        // n: exp(-2 pi i m / n)
-    double2 *G = nullptr;         // n^3: the deconvolved model at k mod n, then its FFT
-    void *fft = nullptr;          // hipfftHandle of the n^3 Z2Z transform
+    double2 *G = nullptr;         // trig table and the two half-transformed models (dft.hip)
     bool loaded = false;
     // type-1 (adjoint) state, allocated on first use
     double *acc = nullptr;        // (np)^3 FP64 spreading grid
@@ -25,6 +24,13 @@ struct mtip_plan {
     double2 *a2 = nullptr;        // np * K * (h + 1)
     bool spread_open = false;     // mtip_plan_spread_begin called
 };
+
+namespace mtip {
+
+// Fine grid of a plan from its model (dft.hip).
+int grid_from_model(mtip_plan *p, const float *ac, hipStream_t st);
+
+}  // namespace mtip
 
 namespace {
 
