@@ -237,6 +237,22 @@ int mtip_merge_combine(const double *y_ups, const double *y_reg, const double *u
                        double *out, void *stream);
 
 /*
+ * Either convolution of the operator without FFTs, 2 <= M <= M_ups <= 320:
+ *   out = scale s . crop(K * pad(s . u)) + coef base,
+ * K a real kernel, cyclic on the M_ups grid (M for the regulariser), with spectrum:
+ * device complex double (M_ups / 2 + 1, M_ups, M_ups), its forward transform with
+ * the first axis halved; support may be NULL for 1; base may be out.  work: at
+ * least mtip_merge_conv_workspace_size(M, M_ups) bytes (0 = sizes not taken),
+ * 16-byte aligned; mtip_merge_conv_prepare fills its tables once per workspace.
+ * One call at a time per workspace.
+ */
+size_t mtip_merge_conv_workspace_size(int M, int M_ups);
+int mtip_merge_conv_prepare(int M, int M_ups, void *work, size_t work_bytes, void *stream);
+int mtip_merge_conv(const double *u, const double *support, const void *spectrum, int M, int M_ups,
+                    double scale, double coef, const double *base, void *work, size_t work_bytes,
+                    double *out, void *stream);
+
+/*
  * Conjugate-gradient steps of cupyx/scipy cg (:211-212) with the step
  * lengths on the device: mtip_dot writes a . b to *out (two fixed-order
  * reduction passes, workspace of mtip_dot_workspace_size() bytes);

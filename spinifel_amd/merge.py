@@ -16,8 +16,10 @@ Where the work runs:
     term at M with the support) -- libmtip's spreading kernel and transform
     passes, positions formed on the fly from the quaternions (no H, K, L
     arrays), the images resident in HBM as FP32;
-  * the per-iteration FFTs (the convolution on the M_ups^3 grid and the
-    Fourier regulariser on M^3) -- rocFFT through torch.fft, in FP64, as
+  * per iteration, the convolution on the M_ups^3 grid -- libmtip's transforms
+    by DFT matrices, which neither store nor transform the padding (90 us at
+    M = 81, M_ups = 162; an FFT pair with its copies took 220 us) -- and the
+    Fourier regulariser on M^3 -- rocFFT through torch.fft, in FP64, as
     real-to-complex transforms: every operand is real and every product
     Hermitian, so irfftn(rfftn(.) * half-spectrum) equals the reference's
     real part of ifftn(fftn(.) * spectrum) (the regulariser's mask is
@@ -168,6 +170,25 @@ def cg_fused(matvec, b, x0, maxiter, tol=1e-5, callback=None):
     return x, info, it
 
 
+class _Convolution:
+    """out = scale s . crop(K * pad(s . u)) + coef base by libmtip's pruned transforms,
+    K given by its spectrum (n / 2 + 1, n, n), with a workspace of its own."""
+
+    def __init__(self, lib, M, n, spectrum, device):
+        self.lib, self.M, self.n, self.spectrum = lib, M, n, spectrum
+        self.work = torch.empty(int(lib.mtip_merge_conv_workspace_size(M, n)) // 8,
+                                dtype=torch.float64, device=device)
+        _lib.check(lib.mtip_merge_conv_prepare(M, n, engine._ptr(self.work), self.work.numel() * 8,
+                                               engine._stream()), "mtip_merge_conv_prepare")
+
+    def __call__(self, u, support, scale, coef, base, out):
+        P = engine._ptr
+        _lib.check(self.lib.mtip_merge_conv(P(u), P(support), P(self.spectrum), self.M, self.n,
+                                            scale, coef, P(base), P(self.work),
+                                            self.work.numel() * 8, P(out), engine._stream()),
+                   "mtip_merge_conv")
+
+
 class Merge:
     """spinifel/sequential/autocorrelation.py:35-225 on the GPU."""
 
@@ -212,7 +233,6 @@ class Merge:
         self._plan_ups = get_plan(self.M_ups, self.eps, self.device.index or 0)
         # zero-padded operand of the convolution; only [:M]^3 is ever written
         self._ups = torch.zeros((self.M_ups,) * 3, dtype=torch.float64, device=self.device)
-        self._us = torch.empty((self.M,) * 3, dtype=torch.float64, device=self.device)
 
         def callback(xk):
             callback.counter += 1
@@ -285,31 +305,27 @@ class Merge:
         ugrid_conv = self._plan_ups.adjoint_points(x, y, z, values=None,
                                                    out_scale=1.0 / self.M_ups ** 3, spatial=False)
         del x, y, z
-        F_half = torch.fft.rfftn(torch.fft.ifftshift(ugrid_conv)) / self.M ** 3
-
-        lib = _lib.load()
-        P = engine._ptr
+        conv = torch.fft.ifftshift(ugrid_conv) / self.M ** 3
+        del ugrid_conv
+        # the real kernel's spectrum, halved along the first axis
+        F = torch.fft.fftn(torch.fft.rfft(conv, dim=0), dim=(1, 2)).contiguous()
+        del conv
+        M = self.M
         sup = ac_support.contiguous()
+        data = _Convolution(_lib.load(), M, self.M_ups, F, self.device)
 
         def W_matvec(uvect):
             # the same operator as core_problem_convolution + rlambda u +
-            # flambda fourier_reg, with the padding and the recombination in
-            # two kernels around the four FFTs
-            M, Mu = self.M, self.M_ups
+            # flambda fourier_reg.  The regulariser keeps its FFT pair on M^3: with
+            # its weight of 1e3 it decides how rounding carries through the
+            # unconverged iterations, which the data term's rounding does not touch
             u = uvect.contiguous()
-            st = engine._stream()
-            _lib.check(lib.mtip_merge_pad(P(u), P(sup), M, Mu, P(self._ups), P(self._us), st),
-                       "mtip_merge_pad")
-            X = torch.fft.rfftn(self._ups)
-            X *= F_half
-            y_ups = torch.fft.irfftn(X, s=(Mu,) * 3).contiguous()
-            R = torch.fft.rfftn(self._us)
+            R = torch.fft.rfftn(u.view(M, M, M) * sup)
             R *= self._reg_mask
-            y_reg = torch.fft.irfftn(R, s=(M,) * 3).contiguous()
+            y_reg = torch.fft.irfftn(R, s=(M, M, M))
             out = torch.empty(M ** 3, dtype=torch.float64, device=self.device)
-            _lib.check(lib.mtip_merge_combine(P(y_ups), P(y_reg), P(u), P(sup), M, Mu,
-                                              float(self.rlambda), float(self.flambda), P(out),
-                                              st), "mtip_merge_combine")
+            data(u, sup, 1.0, float(self.rlambda), u, out)
+            out.view(M, M, M).addcmul_(y_reg, sup, value=float(self.flambda))
             return out
 
         xd, yd, zd, vd = data_pts
