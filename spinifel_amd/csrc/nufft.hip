@@ -11,6 +11,7 @@
 // (n + 2 pad)^3 values, indices l in [-n/2 - pad, n/2 + pad), evaluated
 // directly at the padded indices so no wrap is needed while interpolating.
 #include <math.h>
+#include <algorithm>
 #include <vector>
 
 #include "nufft_shared.h"
@@ -366,7 +367,8 @@ __global__ __launch_bounds__(256, 3) void k_slices_lds(GridView gv, const double
                                                     float *__restrict__ out, int64_t ld_out,
                                                     uint16_t *__restrict__ out_bf16,
                                                     double *__restrict__ row_sum,
-                                                    double *__restrict__ row_sumsq, int *bad)
+                                                    double *__restrict__ row_sumsq, int *bad,
+                                                    int64_t trips)
 {
     using PT = PairTaps<W>;
     constexpr int GP = PT::GP, NS = PT::NS, PPW = 64 / GP;
@@ -406,7 +408,10 @@ __global__ __launch_bounds__(256, 3) void k_slices_lds(GridView gv, const double
     uint16_t *brow = out_bf16 ? out_bf16 + o * ld_out : nullptr;
     double sum = 0.0, sumsq = 0.0;
     int nbad = 0;
-    const int64_t n_slots = order ? n_order : N_p;
+    // this workgroup's trips of 256 slots: all of the orientation's, or its share of them
+    const int64_t n_all = order ? n_order : N_p;
+    const int64_t first_slot = (int64_t)blockIdx.y * trips * 256;
+    const int64_t n_slots = n_all < first_slot + trips * 256 ? n_all : first_slot + trips * 256;
 
     // pixel index and q-vector of this thread's point, prefetched one trip ahead
     // (and the pixel index two trips ahead) so their latency hides behind taps
@@ -414,7 +419,7 @@ __global__ __launch_bounds__(256, 3) void k_slices_lds(GridView gv, const double
         if (order) return (k < n_order) ? order[k] : -1;
         return (k < N_p) ? (int)k : -1;
     };
-    int pix_n = pixel_at(tid);
+    int pix_n = pixel_at(first_slot + tid);
     double qx_n = 0.0, qy_n = 0.0, qz_n = 0.0;
     {
         const int pp = pix_n >= 0 ? pix_n : 0;
@@ -422,9 +427,9 @@ __global__ __launch_bounds__(256, 3) void k_slices_lds(GridView gv, const double
         qy_n = q[N_p + pp];
         qz_n = q[2 * N_p + pp];
     }
-    int pix_nn = pixel_at(256 + tid);
+    int pix_nn = pixel_at(first_slot + 256 + tid);
 
-    for (int64_t tb = 0; tb < n_slots; tb += 256) {
+    for (int64_t tb = first_slot; tb < n_slots; tb += 256) {
         // ---- geometry of this thread's point
         const int pix = pix_n;
         const double x = qx_n, y = qy_n, z = qz_n;
@@ -635,19 +640,62 @@ __global__ __launch_bounds__(256) void k_positions(const double *__restrict__ qu
     L[k] = (ri[2][0] * qx + ri[2][1] * qy + ri[2][2] * qz) * scale;
 }
 
+// FP64 sum and sum of squares of rows of float32, a workgroup each: n values, or
+// those of the n slots of `order` (-1 = none).
+__global__ __launch_bounds__(256) void k_row_sums(const float *__restrict__ v, int64_t ld, int64_t n,
+                                                  const int32_t *__restrict__ order,
+                                                  double *__restrict__ row_sum,
+                                                  double *__restrict__ row_sumsq)
+{
+    __shared__ double s_red[4];
+    const float *row = v + (int64_t)blockIdx.x * ld;
+    double sum = 0.0, sumsq = 0.0;
+#pragma unroll 8
+    for (int64_t i = threadIdx.x; i < n; i += 256) {
+        const int64_t j = order ? order[i] : i;
+        const double x = j >= 0 ? row[j] : 0.f;
+        sum += x;
+        sumsq += x * x;
+    }
+    const double ts = block_sum_f64(sum, s_red), tq = block_sum_f64(sumsq, s_red);
+    if (threadIdx.x == 0) {
+        if (row_sum) row_sum[blockIdx.x] = ts;
+        if (row_sumsq) row_sumsq[blockIdx.x] = tq;
+    }
+}
+
 template <int W>
 void launch_slices(const GridView &gv, const double *quats, int64_t N_o, const double *q,
                    int64_t N_p, const int32_t *order, int64_t n_order, int tile,
                    const int32_t *orient_order, double gscale, float *out, int64_t ld,
                    uint16_t *obf, double *rs, double *rq, int *bad, hipStream_t st)
 {
+    // Workgroups an orientation: one with many orientations; below 4,096 (five rounds of
+    // the 768 workgroups that fit the chip) 8 trips each, fewer where that leaves less
+    // than two workgroups a place.  One workgroup an orientation leaves CUs idle in the
+    // last round, and with few orientations: 1,000 x 16k points (64 trips) 1,065 us
+    // whole, 918 at 8 trips a part, 953 at 4, 962 at 1; 1,009 x 14k at M = 121 1,553 and
+    // 1,320; 50 x 1,024 points 79 and 55 us.  The row sums then take a pass of their own
+    // over the values (in these figures), which costs 10,000 x 16k points in float32 and
+    // bf16 more than the last round does (the step 12.0 against 11.85 ms).
+    const int64_t trips = mtip::ceil_div(order ? n_order : N_p, 256);
+    const int64_t most =
+        N_o >= 4096 ? trips : std::max<int64_t>(1, std::min<int64_t>(8, trips * N_o / 1536));
+    const int64_t parts = std::min<int64_t>(mtip::ceil_div(trips, most), 65535);
+    const int64_t per = mtip::ceil_div(trips, parts);
+    const dim3 wgs((unsigned)N_o, (unsigned)mtip::ceil_div(trips, per));
+    const bool split = wgs.y > 1;
 #define MTIP_SLICES_TP(T)                                                                     \
-    hipLaunchKernelGGL((k_slices_lds<W, T>), dim3((unsigned)N_o), dim3(256), 0, st, gv, quats, q, \
-                       N_p, order, n_order, orient_order, gscale, out, ld, obf, rs, rq, bad)
+    hipLaunchKernelGGL((k_slices_lds<W, T>), wgs, dim3(256), 0, st, gv, quats, q, N_p, order, n_order, \
+                       orient_order, gscale, out, ld, obf, split ? nullptr : rs, split ? nullptr : rq, \
+                       bad, per)
     if (tile == 64) MTIP_SLICES_TP(64);
     else if (tile == 128) MTIP_SLICES_TP(128);
     else MTIP_SLICES_TP(256);
 #undef MTIP_SLICES_TP
+    if (split && (rs || rq))
+        hipLaunchKernelGGL(k_row_sums, dim3((unsigned)N_o), dim3(256), 0, st, out, ld,
+                           order ? n_order : N_p, order, rs, rq);
 }
 
 template <int W>
