@@ -10,14 +10,11 @@
 // Only Re f_k is produced: every caller keeps the real part (spinifel's
 // adjoint with use_recip_sym, autocorrelation.py:123-124 and
 // extern/nufft_ext.py:323-324).  For real c the grid b is real, so
-// f~(-k) = conj f~(k); the passes transform the fast axis to k3 in [0, M/2]
-// only and the last pass writes each (k1, k2, k3 > 0) result also at
-// (-k1, -k2, -k3).
+// f~(-k) = conj f~(k): the passes (dft.hip) keep k1 in [0, M/2] only.
 //
 // b lives on the padded grid of the plan (indices l in [-n/2 - pad,
-// n/2 + pad)), so windows never wrap; the passes sum over the padded indices,
-// which folds the pads onto the periodic grid because exp(2 pi i k l / n)
-// has period n in l.
+// n/2 + pad)), so windows never wrap; the passes add up the padded copies of a
+// point, because exp(2 pi i k l / n) has period n in l.
 //
 // Spreading: a workgroup takes a tile of points (a detector tile of one
 // orientation, or 128 consecutive caller points), bounds the union of their
@@ -31,8 +28,6 @@
 #include "nufft_shared.h"
 
 namespace {
-
-constexpr int kAdjOch = 8;         // outputs per thread of a transform pass
 
 __global__ __launch_bounds__(256) void k_zero_f64(double *__restrict__ p, int64_t n)
 {
@@ -293,99 +288,6 @@ __global__ __launch_bounds__(256, 3) void k_spread(GridView gv, double *__restri
     if (nbad && bad) atomicAdd(bad, nbad);
 }
 
-// One separable pass of the transform back to modes:
-//   out[a][kk][c] = sum_{o < L} in(a, o, c) exp(+2 pi i k l / n),
-//   k = kk + k_lo (kk < NK), l = o - off.
-// MODE 0: real input, complex output.  MODE 1: complex -> complex.
-// MODE 2 (last pass, axis 0, A = 1, c = k2i (h + 1) + k3): writes
-//   out_r[i1][i2][i3] = Re(.) dinv(k1) dinv(k2) dinv(k3) scale support[i]
-// at (k1, k2, k3) and, for k3 > 0, at (-k1, -k2, -k3), where i_d = k_d + M/2.
-template <int MODE>
-__global__ __launch_bounds__(256) void k_adj_pass(const double *__restrict__ in_r,
-                                                  const double2 *__restrict__ in_c,
-                                                  double2 *__restrict__ out_c,
-                                                  const double2 *__restrict__ tw, int n, int L,
-                                                  int off, int NK, int k_lo, int64_t A, int64_t C,
-                                                  double *__restrict__ out_r,
-                                                  const double *__restrict__ dinv, int h, int M,
-                                                  const double *__restrict__ support, double scale)
-{
-    extern __shared__ double2 s_tw[];
-    for (int i = threadIdx.x; i < n; i += blockDim.x) s_tw[i] = tw[i];
-    __syncthreads();
-
-    const int nchunk = (NK + kAdjOch - 1) / kAdjOch;
-    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= A * nchunk * C) return;
-    const int64_t c = t % C;
-    const int64_t r = t / C;
-    const int chunk = (int)(r % nchunk);
-    const int64_t a = r / nchunk;
-    const int kk0 = chunk * kAdjOch;
-
-    // phase index (k l) mod n of each output, advanced by k mod n per input
-    const int l0 = ((-off) % n + n) % n;
-    int idx[kAdjOch], step[kAdjOch];
-#pragma unroll
-    for (int j = 0; j < kAdjOch; ++j) {
-        const int k = kk0 + j + k_lo;
-        step[j] = ((k % n) + n) % n;
-        idx[j] = (int)(((int64_t)step[j] * l0) % n);
-    }
-    double acc_re[kAdjOch], acc_im[kAdjOch];
-#pragma unroll
-    for (int j = 0; j < kAdjOch; ++j) acc_re[j] = acc_im[j] = 0.0;
-
-    for (int o = 0; o < L; ++o) {
-        double vr, vi = 0.0;
-        if (MODE == 0) {
-            vr = in_r[a * L + o];
-        } else {
-            const double2 v = in_c[(a * L + o) * C + c];
-            vr = v.x;
-            vi = v.y;
-        }
-#pragma unroll
-        for (int j = 0; j < kAdjOch; ++j) {
-            // tw = exp(-i theta): exp(+i theta) = (tw.x, -tw.y)
-            const double2 e = s_tw[idx[j]];
-            const double cs = e.x, sn = -e.y;
-            if (MODE == 0) {
-                acc_re[j] = fma(vr, cs, acc_re[j]);
-                acc_im[j] = fma(vr, sn, acc_im[j]);
-            } else {
-                acc_re[j] = fma(vr, cs, fma(-vi, sn, acc_re[j]));
-                acc_im[j] = fma(vr, sn, fma(vi, cs, acc_im[j]));
-            }
-            idx[j] += step[j];
-            idx[j] -= idx[j] >= n ? n : 0;
-        }
-    }
-#pragma unroll
-    for (int j = 0; j < kAdjOch; ++j) {
-        const int kk = kk0 + j;
-        if (kk >= NK) break;
-        if (MODE != 2) {
-            out_c[(a * NK + kk) * C + c] = make_double2(acc_re[j], acc_im[j]);
-        } else {
-            const int k1 = kk + k_lo;
-            const int hp1 = h + 1;
-            const int k2 = (int)(c / hp1) - h, k3 = (int)(c % hp1);
-            const double val =
-                acc_re[j] * dinv[k1 + h] * dinv[k2 + h] * dinv[k3 + h] * scale;
-            const int lo = -(M / 2), hi = (M - 1) / 2;
-            if (k1 <= hi && k2 <= hi && k3 <= hi) {
-                const int64_t i = ((int64_t)(k1 - lo) * M + (k2 - lo)) * M + (k3 - lo);
-                out_r[i] = support ? val * support[i] : val;
-            }
-            if (k3 > 0 && -k1 >= lo && -k1 <= hi && -k2 >= lo && -k2 <= hi && -k3 >= lo) {
-                const int64_t i = ((int64_t)(-k1 - lo) * M + (-k2 - lo)) * M + (-k3 - lo);
-                out_r[i] = support ? val * support[i] : val;
-            }
-        }
-    }
-}
-
 template <int W>
 void launch_spread(const GridView &gv, double *acc, int geom, const double *quats, int64_t N_o,
                    const double *q, int64_t N_p, const int32_t *order, int64_t n_order, int tile,
@@ -418,12 +320,15 @@ extern "C" int mtip_plan_spread_begin(mtip_plan *p, void *stream)
         hipError_t err = hipMalloc(&p->acc, n_acc * sizeof(double));
         if (err == hipSuccess) err = hipMalloc(&p->a1, n_a1 * sizeof(double2));
         if (err == hipSuccess) err = hipMalloc(&p->a2, n_a2 * sizeof(double2));
+        if (err == hipSuccess) err = hipMalloc(&p->at, mtip::modes_table_entries(p) * sizeof(double2));
+        if (err == hipSuccess) err = mtip::modes_table(p, (hipStream_t)stream);
         if (err != hipSuccess) {
             (void)hipFree(p->acc);
             (void)hipFree(p->a1);
             (void)hipFree(p->a2);
+            (void)hipFree(p->at);
             p->acc = nullptr;
-            p->a1 = p->a2 = nullptr;
+            p->a1 = p->a2 = p->at = nullptr;
             return mtip::fail(err == hipErrorOutOfMemory ? MTIP_ERR_NOMEM : MTIP_ERR_HIP,
                               std::string("mtip_plan_spread_begin: ") + hipGetErrorString(err));
         }
@@ -501,30 +406,5 @@ extern "C" int mtip_plan_spread_finish(mtip_plan *p, const double *support, doub
                  "mtip_plan_spread_finish: mtip_plan_spread_begin not called");
     MTIP_REQUIRE(std::isfinite(scale), MTIP_ERR_ARG, "mtip_plan_spread_finish: scale not finite");
     DeviceGuard dg(p->device);
-    hipStream_t st = (hipStream_t)stream;
-    const int np = p->np, h = p->h, K = p->K, n = p->n;
-    const int nh = h + 1;
-    const size_t shm = n * sizeof(double2);
-    auto nblk = [](int64_t A, int NK, int64_t C) {
-        return (unsigned)mtip::ceil_div(A * ((NK + kAdjOch - 1) / kAdjOch) * C, 256);
-    };
-    // pass 0: axis 2 (l3 -> k3 in [0, h]), real input [l1 l2][l3]
-    int64_t A = (int64_t)np * np, C = 1;
-    hipLaunchKernelGGL(k_adj_pass<0>, dim3(nblk(A, nh, C)), dim3(256), shm, st, p->acc, nullptr,
-                       p->a1, p->tw, n, np, p->off, nh, 0, A, C, nullptr, nullptr, h, p->M,
-                       nullptr, 0.0);
-    // pass 1: axis 1 (l2 -> k2 in [-h, h]), input [l1][l2][k3]
-    A = np;
-    C = nh;
-    hipLaunchKernelGGL(k_adj_pass<1>, dim3(nblk(A, K, C)), dim3(256), shm, st, nullptr, p->a1,
-                       p->a2, p->tw, n, np, p->off, K, -h, A, C, nullptr, nullptr, h, p->M,
-                       nullptr, 0.0);
-    // pass 2: axis 0 (l1 -> k1 in [-h, h]), input [l1][k2 k3], real output
-    A = 1;
-    C = (int64_t)K * nh;
-    hipLaunchKernelGGL(k_adj_pass<2>, dim3(nblk(A, K, C)), dim3(256), shm, st, nullptr, p->a2,
-                       nullptr, p->tw, n, np, p->off, K, -h, A, C, out, p->dinv, h, p->M, support,
-                       scale);
-    MTIP_HIP_CHECK(hipGetLastError());
-    return MTIP_OK;
+    return mtip::modes_from_grid(p, support, scale, out, (hipStream_t)stream);
 }

@@ -21,6 +21,8 @@
 // 162 1,490 -> 200, 320 11,600 -> 2,080; a plan's first model 1.1 s (the FFT
 // library's setup) -> 0.5 ms, its buffers (M = 121) 250 -> 46 MB.  Convolution at
 // M = 81 on 162^3 points 90 us (FFT pair with its copies 220), M = 121 on 242^3 248.
+// Modes of a spread grid (a thread per 8 outputs with a sincos table in LDS before):
+// 323 us less 250 at M = 81, 1,520 us less at M = 162.
 // Bound: the chain of one workgroup (load, 2 to 40 products, store) more than the
 // matrix cores (12 us of the 85 at M = 121) or the 82 MB written.  One column tile
 // a workgroup beats two (M = 121 97 against 116 us, M = 41 21 against 30, at four
@@ -522,6 +524,141 @@ __global__ __launch_bounds__(512) void k_conv_axis1_inv(const double2 *__restric
     });
 }
 
+// ----------------------------------------------------- spread grid -> modes (type 1)
+//
+// F(k) = sum_l v(l) exp(+i t k l) of the real padded grid (np = n + 2 pad points an
+// axis, point p at l = p - off, cyclic in n), folded over l and -l; modes k1 >= 0
+// only, the others being conjugates.
+
+// Sum of the padded copies of index l (0 <= l < n) of an axis with the given stride.
+__device__ __forceinline__ double folded(const double *v, int64_t stride, int l, int n, int np, int off)
+{
+    double s = 0.0;
+    int p = l + off % n;
+    for (p = p >= n ? p - n : p; p < np; p += n) s += v[p * stride];
+    return s;
+}
+
+// Axis 1: column (p2, p3), outputs k1 in [0, h]; w1[k1][p2][p3].
+template <int NT>
+__global__ __launch_bounds__(512) void k_modes_axis1(const double *__restrict__ acc,
+                                                     const double2 *__restrict__ T, int Cp, int Op,
+                                                     double2 *__restrict__ w1, int h, int n, int np,
+                                                     int off)
+{
+    extern __shared__ double2 s_dft[];
+    const int ncol = np * np, col0 = blockIdx.x * 16, lane = threadIdx.x & 63;
+    dft_stage<false>(s_dft, 16, n / 2 + 1, Cp, [&](int l, int j) {
+        const int c = col0 + j;
+        if (c >= ncol) return make_double2(0.0, 0.0);
+        const double a = folded(acc + c, ncol, l, n, np, off);
+        const double b = l > 0 && 2 * l != n ? folded(acc + c, ncol, n - l, n, np, off) : 0.0;
+        return make_double2(a + b, a - b);
+    });
+    __syncthreads();
+    double4v Cs[NT][1], Ss[NT][1];
+    dft_all<1, NT, false>(s_dft, 16, Cp, T, Op, Cs, Ss);
+    for_tiles<NT>(Cs, Ss, [&](int lt, double4v C, double4v S) {
+        const int c = col0 + (lane & 15);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int k1 = lt * 16 + 4 * r + (lane >> 4);
+            if (c < ncol && k1 <= h) w1[(int64_t)k1 * ncol + c] = make_double2(C[r], S[r]);
+        }
+    });
+}
+
+// Axis 2 of plane k1 (blockIdx.y): column (p3, re / im), outputs k2 in [-h, h];
+// w2[k1][k2][p3].
+template <int NT>
+__global__ __launch_bounds__(512) void k_modes_axis2(const double *__restrict__ w1,
+                                                     const double2 *__restrict__ T, int Cp, int Op,
+                                                     double *__restrict__ w2, int h, int n, int np,
+                                                     int off)
+{
+    extern __shared__ double2 s_dft[];
+    const int ncol = 2 * np, col0 = blockIdx.x * 16, lane = threadIdx.x & 63;
+    const double *in = w1 + (int64_t)blockIdx.y * np * ncol;
+    double *out = w2 + ((int64_t)blockIdx.y * (2 * h + 1) + h) * ncol;
+    dft_stage<false>(s_dft, 16, n / 2 + 1, Cp, [&](int l, int j) {
+        const int c = col0 + j;
+        if (c >= ncol) return make_double2(0.0, 0.0);
+        const double a = folded(in + c, ncol, l, n, np, off);
+        const double b = l > 0 && 2 * l != n ? folded(in + c, ncol, n - l, n, np, off) : 0.0;
+        return make_double2(a + b, a - b);
+    });
+    __syncthreads();
+    double4v Cs[NT][1], Ss[NT][1];
+    dft_all<1, NT, false>(s_dft, 16, Cp, T, Op, Cs, Ss);
+    for_tiles<NT>(Cs, Ss, [&](int lt, double4v C, double4v S) {
+        const int c = col0 + (lane & 15);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            // C +- i S at +-k2: the real part takes -+ the imaginary column's S, the
+            // imaginary part +- the real column's
+            double o = shfl_xor1_f64(S[r]);
+            if (!(c & 1)) o = -o;
+            const int k2 = lt * 16 + 4 * r + (lane >> 4);
+            if (c >= ncol || k2 > h) continue;
+            out[(int64_t)k2 * ncol + c] = C[r] + o;
+            if (k2 > 0) out[(int64_t)-k2 * ncol + c] = C[r] - o;
+        }
+    });
+}
+
+// Axis 3 of rows (k1 >= 0, k2), real part, deconvolved: mode (k1, k2, k3) and, for
+// k1 > 0, (-k1, -k2, -k3), which has the same real part.
+template <int NT>
+__global__ __launch_bounds__(512) void k_modes_axis3(const double2 *__restrict__ w2,
+                                                     const double2 *__restrict__ T, int Cp, int Op,
+                                                     const double *__restrict__ dinv,
+                                                     const double *__restrict__ support, double scale,
+                                                     double *__restrict__ out, int M, int h, int n,
+                                                     int np, int off)
+{
+    extern __shared__ double2 s_dft[];
+    constexpr int pitch = 17;
+    const int K = 2 * h + 1, nrow = (h + 1) * K, row0 = blockIdx.x * 16, lane = threadIdx.x & 63;
+    dft_stage<true>(s_dft, pitch, n / 2 + 1, Cp, [&](int l, int j) {
+        const int r = row0 + j;
+        if (r >= nrow) return make_double2(0.0, 0.0);
+        const double *v = reinterpret_cast<const double *>(w2 + (int64_t)r * np);
+        double e = folded(v, 2, l, n, np, off), o = folded(v + 1, 2, l, n, np, off);
+        if (l > 0 && 2 * l != n) {
+            e += folded(v, 2, n - l, n, np, off);
+            o -= folded(v + 1, 2, n - l, n, np, off);
+        }
+        return make_double2(e, o);
+    });
+    __syncthreads();
+    double4v Cs[NT][1], Ss[NT][1];
+    dft_all<1, NT, true>(s_dft, pitch, Cp, T, Op, Cs, Ss);
+    const int lo = -(M / 2), hi = (M - 1) / 2;
+    for_tiles<NT>(Cs, Ss, [&](int lt, double4v C, double4v S) {
+        const int k = lt * 16 + (lane & 15);
+        if (k > h) return;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int row = row0 + 4 * r + (lane >> 4);
+            if (row >= nrow) continue;
+            const int k1 = row / K, k2 = row - k1 * K - h;
+            auto put = [&](int a, int b, int c, double v) {
+                if (a < lo || a > hi || b < lo || b > hi || c < lo || c > hi) return;
+                const int64_t i = ((int64_t)(a - lo) * M + (b - lo)) * M + (c - lo);
+                out[i] = support ? v * support[i] : v;
+            };
+            const double w = dinv[k1 + h] * dinv[k2 + h] * dinv[k + h] * scale;
+            const double vp = (C[r] - S[r]) * w, vm = (C[r] + S[r]) * w;      // at k3 = k, -k
+            put(k1, k2, k, vp);
+            if (k > 0) put(k1, k2, -k, vm);
+            if (k1 > 0) {
+                put(-k1, -k2, -k, vp);
+                if (k > 0) put(-k1, -k2, k, vm);
+            }
+        }
+    });
+}
+
 int pad_to(int v, int m) { return (v + m - 1) / m * m; }
 
 // Output tiles a wave and waves a workgroup for Op padded outputs: a wave a tile up
@@ -570,6 +707,46 @@ int grid_from_model(mtip_plan *p, const float *ac, hipStream_t st)
     }
     MTIP_HIP_CHECK(hipGetLastError());
     return MTIP_OK;
+}
+
+size_t modes_table_entries(const mtip_plan *p)
+{
+    return (size_t)pad_to(p->n / 2 + 1, 4) * pad_to(p->h + 1, 16);
+}
+
+hipError_t modes_table(const mtip_plan *p, hipStream_t st)
+{
+    hipLaunchKernelGGL(k_trig_table, dim3((unsigned)ceil_div(modes_table_entries(p), 256)), dim3(256), 0, st,
+                       p->at, p->n / 2 + 1, pad_to(p->n / 2 + 1, 4), p->h + 1, pad_to(p->h + 1, 16), p->n);
+    return hipGetLastError();
+}
+
+int modes_from_grid(mtip_plan *p, const double *support, double scale, double *out, hipStream_t st)
+{
+    const int h = p->h, n = p->n, np = p->np, nh = h + 1;
+    const int Cp = pad_to(n / 2 + 1, 4), Op = pad_to(nh, 16);
+    const size_t lds = (size_t)Cp * 16 * sizeof(double2), lds3 = (size_t)Cp * 17 * sizeof(double2);
+    const dim3 block(64 * waves_of(Op));
+    auto run = [&](auto ntc) -> int {
+        constexpr int NT = decltype(ntc)::value;
+        if (lds3 > 65536)       // M > 237
+            for (const void *f : {reinterpret_cast<const void *>(&k_modes_axis1<NT>),
+                                  reinterpret_cast<const void *>(&k_modes_axis2<NT>),
+                                  reinterpret_cast<const void *>(&k_modes_axis3<NT>)})
+                MTIP_HIP_CHECK(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds3));
+        hipLaunchKernelGGL((k_modes_axis1<NT>), dim3((unsigned)ceil_div((int64_t)np * np, 16)), block, lds,
+                           st, p->acc, p->at, Cp, Op, p->a1, h, n, np, p->off);
+        hipLaunchKernelGGL((k_modes_axis2<NT>), dim3((unsigned)ceil_div(2 * np, 16), nh), block, lds, st,
+                           (const double *)p->a1, p->at, Cp, Op, (double *)p->a2, h, n, np, p->off);
+        hipLaunchKernelGGL((k_modes_axis3<NT>), dim3((unsigned)ceil_div((int64_t)nh * p->K, 16)), block,
+                           lds3, st, p->a2, p->at, Cp, Op, p->dinv, support, scale, out, p->M, h, n, np,
+                           p->off);
+        MTIP_HIP_CHECK(hipGetLastError());
+        return MTIP_OK;
+    };
+    // up to 11 tiles (M <= 320)
+    if (tiles_a_wave(Op) == 1) return run(std::integral_constant<int, 1>{});
+    return run(std::integral_constant<int, 2>{});
 }
 
 }  // namespace mtip

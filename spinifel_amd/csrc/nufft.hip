@@ -73,18 +73,6 @@ double es_phi_host(double z, int w, double beta)
     return v > 0.0 ? exp(beta * (sqrt(v) - 1.0)) : 0.0;
 }
 
-// ------------------------------------------------------------ fine grid
-
-__global__ void k_twiddle(double2 *tw, int n)
-{
-    int m = blockIdx.x * blockDim.x + threadIdx.x;
-    if (m < n) {
-        double s, c;
-        sincospi(2.0 * (double)m / (double)n, &s, &c);
-        tw[m] = make_double2(c, -s);
-    }
-}
-
 // ------------------------------------------------------------ interpolation
 //
 // Lane layout: a group of G lanes (G = 4, 8 or 16 >= w) interpolates one
@@ -753,13 +741,8 @@ extern "C" int mtip_plan_create(int M, double eps, int device, mtip_plan **out)
     size_t ng = (size_t)p->np * p->np * p->np;
     hipError_t err = hipMalloc(&p->grid, ng * sizeof(float));
     if (err == hipSuccess) err = hipMalloc(&p->dinv, p->K * sizeof(double));
-    if (err == hipSuccess) err = hipMalloc(&p->tw, p->n * sizeof(double2));
     if (err == hipSuccess)
         err = hipMemcpy(p->dinv, dinv.data(), p->K * sizeof(double), hipMemcpyHostToDevice);
-    if (err == hipSuccess) {
-        hipLaunchKernelGGL(k_twiddle, dim3((p->n + 255) / 256), dim3(256), 0, 0, p->tw, p->n);
-        err = hipGetLastError();
-    }
     if (err == hipSuccess) err = hipDeviceSynchronize();
     if (err != hipSuccess) {
         std::string msg = std::string("mtip_plan_create: ") + hipGetErrorString(err);
@@ -777,11 +760,11 @@ extern "C" int mtip_plan_destroy(mtip_plan *p)
     DeviceGuard dg(p->device);
     (void)hipFree(p->grid);
     (void)hipFree(p->dinv);
-    (void)hipFree(p->tw);
     (void)hipFree(p->G);
     (void)hipFree(p->acc);
     (void)hipFree(p->a1);
     (void)hipFree(p->a2);
+    (void)hipFree(p->at);
     delete p;
     return MTIP_OK;
 }
