@@ -51,6 +51,14 @@ __global__ __launch_bounds__(256) void k_zero_f64(double *__restrict__ p, int64_
 // the window (lane = row * W + element), so no two lanes ever update one cell
 // at once and a wave's LDS accesses complete in issue order.  A box beyond
 // kBoxCap sends the same per-lane taps to the FP64 grid as global atomics.
+//
+// Bound: instruction issue of the walk (about 50 instructions a point and wave) where
+// the values are dense, the chain of a tile (geometry, weights, walk, box pass) where
+// most are zero.  Points of value zero are taken out before the walk (photon images at
+// 0.1 a pixel: one in ten stays), a tile's points are read while the one before it is
+// spread, the box is cleared by the pass that reads it and that pass keeps four reads
+// in flight: 1,000 images x 16,384 pixels at M = 81, 0.1 photons a pixel, 2,010 -> 862
+// us; dense values 8.7 -> 7.1 ms; 16.4 M ordered points of ones 5.7 -> 4.8 ms.
 template <int W, int TP>
 __global__ __launch_bounds__(256, 3) void k_spread(GridView gv, double *__restrict__ acc, int geom,
                                                  const double *__restrict__ quats,
@@ -70,12 +78,12 @@ __global__ __launch_bounds__(256, 3) void k_spread(GridView gv, double *__restri
     constexpr bool PRE = TP <= 128;
     constexpr int NW = 3 * W;
     constexpr int CAP = PRE ? kBoxCap - TP * NW : kBoxCap;
-    __shared__ float s_box[CAP];
+    __shared__ __align__(16) float s_box[CAP];
     __shared__ float s_w[PRE ? TP * NW : 1];
     __shared__ int s_base[TP];          // window corner: box-local or padded-grid index, -1 none
     __shared__ int s_xc[TP];            // box-local x of the corner
     __shared__ float4 s_pt[TP];         // fractional offsets tx, ty, tz and the value
-    __shared__ int s_red_i[4][6];
+    __shared__ int s_red_i[4][7];
     __shared__ double s_ri[9];
 
     const int tid = threadIdx.x, lane = tid & 63;
@@ -98,6 +106,28 @@ __global__ __launch_bounds__(256, 3) void k_spread(GridView gv, double *__restri
     const int64_t n_slots =
         geom == GEOM_POINTS ? TP : (order ? n_order : mtip::ceil_div(N_p, TP) * TP);
 
+    // the pixel of this thread's slot; slots of GEOM_ROTATE are read ahead, the pixel
+    // index two tiles and its q-vector and value one tile, behind the taps
+    auto pixel_at = [&](int64_t k) -> int64_t {
+        if (geom == GEOM_POINTS || tid >= TP) return -1;
+        return order ? (k < n_order ? (int64_t)order[k] : -1) : (k < N_p ? k : -1);
+    };
+    int64_t pix_n = pixel_at(tid), pix_nn = pixel_at(TP + tid);
+    double x_n = 0.0, y_n = 0.0, z_n = 0.0;
+    float v_n = 0.f;
+    auto fetch = [&] {
+        if (pix_n >= 0) {
+            x_n = q[pix_n];
+            y_n = q[N_p + pix_n];
+            z_n = q[2 * N_p + pix_n];
+            v_n = vals ? vals[o * ld_v + pix_n] : 1.f;
+        }
+    };
+    fetch();
+    // the box is zero between tiles: the last pass over it leaves it so
+    for (int k = tid; k < CAP / 4; k += 256)
+        reinterpret_cast<float4 *>(s_box)[k] = make_float4(0.f, 0.f, 0.f, 0.f);
+
     for (int64_t tb = 0; tb < n_slots; tb += TP) {
         // ---- this thread's point (threads < TP)
         bool ok = false;
@@ -105,7 +135,6 @@ __global__ __launch_bounds__(256, 3) void k_spread(GridView gv, double *__restri
         int ijk[3] = {0, 0, 0};
         float t[3] = {0.f, 0.f, 0.f};
         if (tid < TP) {
-            const int64_t k = tb + tid;
             double X0 = 0.0, X1 = 0.0, X2 = 0.0;
             bool have = false;
             if (geom == GEOM_POINTS) {
@@ -117,17 +146,12 @@ __global__ __launch_bounds__(256, 3) void k_spread(GridView gv, double *__restri
                     X2 = pz[j] * gscale;
                     v = vals ? vals[j] : 1.f;
                 }
-            } else {
-                const int64_t pix = order ? (k < n_order ? (int64_t)order[k] : -1)
-                                          : (k < N_p ? k : -1);
-                if (pix >= 0) {
-                    have = true;
-                    const double x = q[pix], y = q[N_p + pix], z = q[2 * N_p + pix];
-                    X0 = (s_ri[0] * x + s_ri[1] * y + s_ri[2] * z) * gscale;
-                    X1 = (s_ri[3] * x + s_ri[4] * y + s_ri[5] * z) * gscale;
-                    X2 = (s_ri[6] * x + s_ri[7] * y + s_ri[8] * z) * gscale;
-                    v = vals ? vals[o * ld_v + pix] : 1.f;
-                }
+            } else if (pix_n >= 0) {
+                have = true;
+                X0 = (s_ri[0] * x_n + s_ri[1] * y_n + s_ri[2] * z_n) * gscale;
+                X1 = (s_ri[3] * x_n + s_ri[4] * y_n + s_ri[5] * z_n) * gscale;
+                X2 = (s_ri[6] * x_n + s_ri[7] * y_n + s_ri[8] * z_n) * gscale;
+                v = v_n;
             }
             if (have) {
                 ok = point_corner<W>(gv, X0, X1, X2, ijk, t);
@@ -135,15 +159,21 @@ __global__ __launch_bounds__(256, 3) void k_spread(GridView gv, double *__restri
                 if (v == 0.f) ok = false;     // contributes nothing
             }
         }
-        // ---- box of the tile's windows (block min / max)
+        pix_n = pix_nn;
+        fetch();
+        pix_nn = pixel_at(tb + 2 * TP + tid);
+        // ---- box of the tile's windows (block min / max) and the points that count
+        const uint64_t on = __ballot(ok);
         {
             int r[6] = {ok ? ijk[0] : 0x7fffffff, ok ? ijk[1] : 0x7fffffff, ok ? ijk[2] : 0x7fffffff,
                         ok ? -ijk[0] : 0x7fffffff, ok ? -ijk[1] : 0x7fffffff, ok ? -ijk[2] : 0x7fffffff};
 #pragma unroll
             for (int e = 0; e < 6; ++e) r[e] = wave_min_i(r[e]);
-            if (lane == 0)
+            if (lane == 0) {
 #pragma unroll
                 for (int e = 0; e < 6; ++e) s_red_i[wave][e] = r[e];
+                s_red_i[wave][6] = __popcll(on);
+            }
         }
         __syncthreads();
         int lo[3], hi[3];
@@ -153,24 +183,30 @@ __global__ __launch_bounds__(256, 3) void k_spread(GridView gv, double *__restri
             hi[e] = -min(min(s_red_i[0][e + 3], s_red_i[1][e + 3]),
                          min(s_red_i[2][e + 3], s_red_i[3][e + 3]));
         }
-        if (lo[0] == 0x7fffffff) {
+        int n_act = 0, before = 0;
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+            if (w == wave) before = n_act;
+            n_act += s_red_i[w][6];
+        }
+        if (n_act == 0) {
             __syncthreads();     // s_red_i is rewritten by the next tile
             continue;
         }
         const int bx = hi[0] - lo[0] + W, by = hi[1] - lo[1] + W, bz = hi[2] - lo[2] + W;
         const bool staged = bx * by * bz <= CAP;
         const int ncell = staged ? bx * by * bz : 0;
-        if (tid < TP) {
-            s_base[tid] = !ok ? -1
-                        : staged ? ((ijk[0] - lo[0]) * by + (ijk[1] - lo[1])) * bz + (ijk[2] - lo[2])
-                                 : (ijk[0] * np + ijk[1]) * np + ijk[2];
-            s_xc[tid] = ijk[0] - lo[0];
-            s_pt[tid] = make_float4(t[0], t[1], t[2], v);
+        if (ok) {
+            // the points that count, in their order
+            const int i = before + __popcll(on & ((1ull << lane) - 1));
+            s_base[i] = staged ? ((ijk[0] - lo[0]) * by + (ijk[1] - lo[1])) * bz + (ijk[2] - lo[2])
+                               : (ijk[0] * np + ijk[1]) * np + ijk[2];
+            s_xc[i] = ijk[0] - lo[0];
+            s_pt[i] = make_float4(t[0], t[1], t[2], v);
         }
-        for (int k = tid; k < ncell; k += 256) s_box[k] = 0.f;
         __syncthreads();
         if constexpr (PRE) {
-            for (int k = tid; k < TP * NW; k += 256) {
+            for (int k = tid; k < n_act * NW; k += 256) {
                 const int pn = k / NW, r = k - pn * NW, d = r / W, e = r - d * W;
                 const float4 pt = s_pt[pn];
                 const float tt = d == 0 ? pt.x : d == 1 ? pt.y : pt.z;
@@ -179,35 +215,38 @@ __global__ __launch_bounds__(256, 3) void k_spread(GridView gv, double *__restri
             }
             __syncthreads();
         }
-        // ---- taps: every wave walks all TP points, updating its own x planes;
-        // a chunk of 64 points' parameters is read into registers at once and
-        // each point's taken from its lane by readlane (scalar operands).  A
-        // point's planes (a0, a0 + 4, ...) are read together, then added and
-        // written, so one LDS round trip serves them all; with precomputed
-        // weights the next point's are read while this point's planes wait.
+        // ---- taps: every wave walks all the points, updating its own x planes; a
+        // chunk of 64 points' parameters is read into registers at once and each
+        // point's taken from its lane by readlane (scalar operands).  A point's
+        // planes (a0, a0 + 4, ...) are read together, then added and written, so one
+        // LDS round trip serves them all; with precomputed weights the next point's
+        // are read while this point's planes wait.
         const int plane = staged ? by * bz : np * np, rowstride = staged ? bz : np;
         constexpr int NPL = (W + 3) / 4;      // planes per point and wave, at most
-        auto taps = [&](int base, int a0, float pa, const float (&wyz)[NPASS])
+        int lane_off[NPASS];
+        bool pass_on[NPASS];
+#pragma unroll
+        for (int ps = 0; ps < NPASS; ++ps) {
+            const int b = ps * RP + lrow;
+            pass_on[ps] = lane_on && b < W;
+            lane_off[ps] = b * rowstride + lel;
+        }
+        // first: the point's corner in its first plane a0 of this wave
+        auto taps = [&](bool in_box, int first, int a0, const float (&wa)[NPL], const float (&wyz)[NPASS])
             __attribute__((always_inline)) {
 #pragma unroll
             for (int ps = 0; ps < NPASS; ++ps) {
-                const int b = ps * RP + lrow;
-                if (!lane_on || b >= W) continue;
-                const int off = base + b * rowstride + lel + a0 * plane;
-                float wa[NPL];
-#pragma unroll
-                for (int j = 0; j < NPL; ++j)
-                    wa[j] = a0 + 4 * j < W ? __int_as_float(__builtin_amdgcn_readlane(
-                                                 __float_as_int(pa), a0 + 4 * j))
-                                           : 0.f;
-                if (staged) {
+                if (!pass_on[ps]) continue;
+                const int off = first + lane_off[ps];
+                if (in_box) {
                     float cur[NPL];
 #pragma unroll
                     for (int j = 0; j < NPL; ++j)
-                        if (a0 + 4 * j < W) cur[j] = s_box[off + 4 * j * plane];
+                        if (4 * j + 3 < W || a0 + 4 * j < W) cur[j] = s_box[off + 4 * j * plane];
 #pragma unroll
                     for (int j = 0; j < NPL; ++j)
-                        if (a0 + 4 * j < W) s_box[off + 4 * j * plane] = fmaf(wa[j], wyz[ps], cur[j]);
+                        if (4 * j + 3 < W || a0 + 4 * j < W)
+                            s_box[off + 4 * j * plane] = fmaf(wa[j], wyz[ps], cur[j]);
                 } else {
 #pragma unroll
                     for (int j = 0; j < NPL; ++j)
@@ -217,73 +256,93 @@ __global__ __launch_bounds__(256, 3) void k_spread(GridView gv, double *__restri
                 }
             }
         };
+        auto walk = [&](auto boxed) __attribute__((always_inline)) {
+            constexpr bool IN_BOX = decltype(boxed)::value;
 #pragma unroll 1
-        for (int c0 = 0; c0 < TP; c0 += 64) {
-            const int cl = c0 + lane < TP ? c0 + lane : TP - 1;
-            const int r_base = s_base[cl], r_xc = s_xc[cl];
-            const int nc = TP - c0 < 64 ? TP - c0 : 64;
-            if constexpr (PRE) {
-                // weights of point i: x by lane (lanes < W), y by row, z (x value) by element
-                auto load = [&](int i, float &pa, float (&wy)[NPASS], float &wz)
-                    __attribute__((always_inline)) {
-                    const float *wp = s_w + (c0 + i) * NW;
-                    pa = wp[lane < W ? lane : 0];
-                    wz = wp[2 * W + lel];
+            for (int c0 = 0; c0 < n_act; c0 += 64) {
+                const int cl = min(c0 + lane, n_act - 1);
+                const int r_a0 = (wave - s_xc[cl]) & 3;
+                const int r_first = s_base[cl] + r_a0 * plane;
+                const int nc = min(n_act - c0, 64);
+                if constexpr (PRE) {
+                    // weights of point i: the wave's x planes (one address for all
+                    // lanes), y by row, z (x value) by element
+                    auto load = [&](int i, float (&wa)[NPL], float (&wy)[NPASS], float &wz)
+                        __attribute__((always_inline)) {
+                        const float *wp = s_w + (c0 + i) * NW;
+                        const int a0 = __builtin_amdgcn_readlane(r_a0, i);
 #pragma unroll
-                    for (int ps = 0; ps < NPASS; ++ps) {
-                        const int b = ps * RP + lrow;
-                        wy[ps] = wp[W + (b < W ? b : W - 1)];
+                        for (int j = 0; j < NPL; ++j) wa[j] = wp[a0 + 4 * j];    // past W: unused
+                        wz = wp[2 * W + lel];
+#pragma unroll
+                        for (int ps = 0; ps < NPASS; ++ps) {
+                            const int b = ps * RP + lrow;
+                            wy[ps] = wp[W + (b < W ? b : W - 1)];
+                        }
+                    };
+                    float n_wa[NPL], n_wy[NPASS], n_wz;
+                    load(0, n_wa, n_wy, n_wz);
+                    for (int i = 0; i < nc; ++i) {
+                        float wa[NPL], wyz[NPASS];
+#pragma unroll
+                        for (int j = 0; j < NPL; ++j) wa[j] = n_wa[j];
+#pragma unroll
+                        for (int ps = 0; ps < NPASS; ++ps) wyz[ps] = n_wy[ps] * n_wz;
+                        if (i + 1 < nc) load(i + 1, n_wa, n_wy, n_wz);
+                        taps(IN_BOX, __builtin_amdgcn_readlane(r_first, i),
+                             __builtin_amdgcn_readlane(r_a0, i), wa, wyz);
                     }
-                };
-                float n_pa, n_wy[NPASS], n_wz;
-                load(0, n_pa, n_wy, n_wz);
-                for (int i = 0; i < nc; ++i) {
-                    const float pa = n_pa, wz = n_wz;
-                    float wyz[NPASS];
+                } else {
+                    const float4 r_pt = s_pt[cl];
+                    for (int i = 0; i < nc; ++i) {
+                        const float tx = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(r_pt.x), i));
+                        const float ty = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(r_pt.y), i));
+                        const float tz = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(r_pt.z), i));
+                        const float pv = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(r_pt.w), i));
+                        const int a0 = __builtin_amdgcn_readlane(r_a0, i);
+                        // lanes 0 .. W-1 hold the x weights, read back per plane
+                        const float pa = es_phi((float)lane - tx, gv.beta_l2e, gv.c2);
+                        const float wz = es_phi((float)lel - tz, gv.beta_l2e, gv.c2) * pv;
+                        float wa[NPL], wyz[NPASS];
 #pragma unroll
-                    for (int ps = 0; ps < NPASS; ++ps) wyz[ps] = n_wy[ps] * wz;
-                    if (i + 1 < nc) load(i + 1, n_pa, n_wy, n_wz);
-                    const int base = __builtin_amdgcn_readlane(r_base, i);
-                    if (base < 0) continue;
-                    taps(base, (wave - __builtin_amdgcn_readlane(r_xc, i)) & 3, pa, wyz);
-                }
-            } else {
-                const float4 r_pt = s_pt[cl];
-                for (int i = 0; i < nc; ++i) {
-                    const int base = __builtin_amdgcn_readlane(r_base, i);
-                    if (base < 0) continue;
-                    const float tx = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(r_pt.x), i));
-                    const float ty = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(r_pt.y), i));
-                    const float tz = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(r_pt.z), i));
-                    const float pv = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(r_pt.w), i));
-                    // lanes 0 .. W-1 hold the x weights, read back per plane
-                    const float pa = es_phi((float)lane - tx, gv.beta_l2e, gv.c2);
-                    const float wz = es_phi((float)lel - tz, gv.beta_l2e, gv.c2) * pv;
-                    float wyz[NPASS];
+                        for (int j = 0; j < NPL; ++j)
+                            wa[j] = a0 + 4 * j < W ? __int_as_float(__builtin_amdgcn_readlane(
+                                                         __float_as_int(pa), a0 + 4 * j))
+                                                   : 0.f;
 #pragma unroll
-                    for (int ps = 0; ps < NPASS; ++ps)
-                        wyz[ps] = es_phi((float)(ps * RP + lrow) - ty, gv.beta_l2e, gv.c2) * wz;
-                    taps(base, (wave - __builtin_amdgcn_readlane(r_xc, i)) & 3, pa, wyz);
+                        for (int ps = 0; ps < NPASS; ++ps)
+                            wyz[ps] = es_phi((float)(ps * RP + lrow) - ty, gv.beta_l2e, gv.c2) * wz;
+                        taps(IN_BOX, __builtin_amdgcn_readlane(r_first, i), a0, wa, wyz);
+                    }
                 }
             }
-        }
+        };
+        if (staged) walk(std::integral_constant<bool, true>{});
+        else walk(std::integral_constant<bool, false>{});
         __syncthreads();
-        // ---- the box's non-zero cells into the FP64 grid
+        // ---- the box's non-zero cells into the FP64 grid, four reads in flight, and
+        // zero again.  No barrier after it: the next tile's taps come after two
         if (staged) {
             const float inv_bz = 1.0f / (float)bz, inv_by = 1.0f / (float)by;
-            for (int k = tid; k < ncell; k += 256) {
-                const float val = s_box[k];
-                if (val != 0.f) {
-                    // k / bz and r / by for k < 2^16: the float estimates are
-                    // within half a unit of the integer quotient
-                    const int r = (int)(((float)k + 0.5f) * inv_bz), z = k - r * bz;
-                    const int xr = (int)(((float)r + 0.5f) * inv_by), yr = r - xr * by;
-                    unsafeAtomicAdd(acc + ((int64_t)(lo[0] + xr) * np + (lo[1] + yr)) * np + lo[2] + z,
-                                    (double)val);
+            for (int k0 = tid; k0 < ncell; k0 += 1024) {
+                float val[4];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) val[u] = s_box[min(k0 + 256 * u, CAP - 1)];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    const int k = k0 + 256 * u;
+                    if (k < ncell && val[u] != 0.f) {
+                        s_box[k] = 0.f;
+                        // k / bz and r / by for k < 2^16: the float estimates are
+                        // within half a unit of the integer quotient
+                        const int r = (int)(((float)k + 0.5f) * inv_bz), z = k - r * bz;
+                        const int xr = (int)(((float)r + 0.5f) * inv_by), yr = r - xr * by;
+                        unsafeAtomicAdd(acc + ((int64_t)(lo[0] + xr) * np + (lo[1] + yr)) * np + lo[2] + z,
+                                        (double)val[u]);
+                    }
                 }
             }
         }
-        __syncthreads();
     }
     if (nbad && bad) atomicAdd(bad, nbad);
 }
