@@ -16,6 +16,7 @@ Pipeline of one ``match`` (all on one stream, inputs resident in HBM):
 6. ``rescore``              -- FP32 and FP64 full distances of the candidates
 """
 import ctypes
+import math
 import threading
 from dataclasses import dataclass
 from typing import NamedTuple
@@ -184,11 +185,16 @@ def _orient_rank(quats):
 
 def auto_tiling(plan, det_shape):
     """Tiling by rule, without timing: 16 x 16 blocks while a block's fine-grid
-    box fits LDS (fine grids up to ~200 points per edge at 0.9 Nyquist), 8 x 8
-    blocks beyond.  The autotuner (spinifel_amd.autotune) picks by timing."""
+    box fits LDS, which takes pixels no further apart than about 1.4 cells of
+    the fine grid -- n_fine <= 1.6 times the edge of a square detector of as
+    many pixels at 0.9 Nyquist -- and 8 x 8 blocks beyond (measured: 2,000
+    orientations of 32 x 32 pixels, n = 90: 264 us for 8 x 8, 316 for 16 x 16;
+    1,000 of 128 x 128, n = 162: 1,088 and 972; 1,009 of 111 x 128, n = 250:
+    1,202 and 1,720).  The autotuner (spinifel_amd.autotune) picks by timing."""
     if len(tuple(det_shape)) < 2:
         return None
-    return tiling(det_shape, (16, 16) if plan.n_fine <= 200 else (8, 8))
+    edge = math.sqrt(math.prod(int(d) for d in det_shape))
+    return tiling(det_shape, (16, 16) if plan.n_fine <= 1.6 * edge else (8, 8))
 
 
 def auto_spread_tiling(plan, det_shape):
