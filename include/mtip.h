@@ -253,6 +253,21 @@ int mtip_merge_conv(const double *u, const double *support, const void *spectrum
                     double *out, void *stream);
 
 /*
+ * The regulariser's elementwise work between complex transforms of n values (a
+ * complex double each): w = (s u, 0); spectrum *= mask (real);
+ * out += flambda s (scale Re back).
+ * mtip_half_pack / mtip_half_expand: the half spectrum of M^3 real values, M odd,
+ * between spectrum (M, M, M), third axis transformed, and half (M / 2 + 1, M, M), third
+ * axis first; expand fills the other half with the conjugates along that axis.
+ */
+int mtip_half_pack(const void *spectrum, int M, void *half, void *stream);
+int mtip_half_expand(const void *half, int M, void *spectrum, void *stream);
+int mtip_merge_reg_embed(const double *u, const double *support, int64_t n, void *w, void *stream);
+int mtip_merge_reg_mask(void *spectrum, const double *mask, int64_t n, void *stream);
+int mtip_merge_reg_add(const void *back, double scale, const double *support, double flambda,
+                       int64_t n, double *out, void *stream);
+
+/*
  * Conjugate-gradient steps of cupyx/scipy cg (:211-212) with the step
  * lengths on the device: mtip_dot writes a . b to *out (two fixed-order
  * reduction passes, workspace of mtip_dot_workspace_size() bytes);

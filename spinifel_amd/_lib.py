@@ -51,6 +51,11 @@ _SIGS = {
     "mtip_phase_update": (_i32, [_vp, _vp, _vp, _i64, _i32, _f64, _f64, _vp]),
     "mtip_clip_bin": (_i32, [_vp, _i32, _i64, _i32, _i32, _i32, _i32, _i32, _i32, _vp, _vp]),
     "mtip_merge_pad": (_i32, [_vp, _vp, _i32, _i32, _vp, _vp, _vp]),
+    "mtip_half_pack": (_i32, [_vp, _i32, _vp, _vp]),
+    "mtip_half_expand": (_i32, [_vp, _i32, _vp, _vp]),
+    "mtip_merge_reg_embed": (_i32, [_vp, _vp, _i64, _vp, _vp]),
+    "mtip_merge_reg_mask": (_i32, [_vp, _vp, _i64, _vp]),
+    "mtip_merge_reg_add": (_i32, [_vp, _f64, _vp, _f64, _i64, _vp, _vp]),
     "mtip_merge_conv_workspace_size": (_c.c_size_t, [_i32, _i32]),
     "mtip_merge_conv_prepare": (_i32, [_i32, _i32, _vp, _c.c_size_t, _vp]),
     "mtip_merge_conv": (_i32, [_vp, _vp, _vp, _i32, _i32, _f64, _f64, _vp, _vp, _c.c_size_t,

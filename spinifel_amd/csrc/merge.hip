@@ -110,6 +110,79 @@ __global__ __launch_bounds__(256) void k_cg_direction(double *__restrict__ p,
         p[i] = first ? r[i] : r[i] + beta * p[i];
 }
 
+// Half spectrum of M^3 values between its two layouts, M odd: F[i][j][k] with the
+// third axis transformed, all of it, and Y[k][i][j], k < M/2 + 1, whose first two axes
+// the FFT library then takes contiguous.  Its own real-to-complex path makes the same
+// values with one copy more each way and the layouts apart (M = 81: 78 us a pair, 54
+// for the four transforms used here).  64 x 16 tiles through LDS.
+constexpr int kHalfRows = 64, kHalfCols = 16;
+
+__global__ __launch_bounds__(256) void k_half_pack(const double2 *__restrict__ F, int M,
+                                                   double2 *__restrict__ Y)
+{
+    __shared__ double2 s[kHalfCols][kHalfRows + 1];
+    const int h = M / 2 + 1, row0 = blockIdx.x * kHalfRows, k0 = blockIdx.y * kHalfCols;
+    const int64_t rows = (int64_t)M * M;
+    for (int t = threadIdx.x; t < kHalfRows * kHalfCols; t += 256) {
+        const int r = t / kHalfCols, k = t % kHalfCols;
+        if (row0 + r < rows && k0 + k < h) s[k][r] = F[(int64_t)(row0 + r) * M + k0 + k];
+    }
+    __syncthreads();
+    for (int t = threadIdx.x; t < kHalfRows * kHalfCols; t += 256) {
+        const int r = t % kHalfRows, k = t / kHalfRows;
+        if (row0 + r < rows && k0 + k < h) Y[(k0 + k) * rows + row0 + r] = s[k][r];
+    }
+}
+
+__global__ __launch_bounds__(256) void k_half_expand(const double2 *__restrict__ Y, int M,
+                                                     double2 *__restrict__ F)
+{
+    __shared__ double2 s[kHalfCols][kHalfRows + 1];
+    const int h = M / 2 + 1, row0 = blockIdx.x * kHalfRows, k0 = blockIdx.y * kHalfCols;
+    const int64_t rows = (int64_t)M * M;
+    for (int t = threadIdx.x; t < kHalfRows * kHalfCols; t += 256) {
+        const int r = t % kHalfRows, k = t / kHalfRows;
+        if (row0 + r < rows && k0 + k < h) s[k][r] = Y[(k0 + k) * rows + row0 + r];
+    }
+    __syncthreads();
+    for (int t = threadIdx.x; t < kHalfRows * kHalfCols; t += 256) {
+        const int r = t / kHalfCols, k = k0 + t % kHalfCols;
+        if (row0 + r >= rows || k >= h) continue;
+        const double2 v = s[k - k0][r];
+        double2 *f = F + (int64_t)(row0 + r) * M;
+        f[k] = v;
+        if (k > 0) f[M - k] = make_double2(v.x, -v.y);
+    }
+}
+
+// w = (s u, 0)
+__global__ __launch_bounds__(256) void k_reg_embed(const double *__restrict__ u,
+                                                   const double *__restrict__ s, int64_t n,
+                                                   double2 *__restrict__ w)
+{
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) w[i] = make_double2(u[i] * s[i], 0.0);
+}
+
+// X *= m, m real
+__global__ __launch_bounds__(256) void k_reg_mask(double2 *__restrict__ X,
+                                                  const double *__restrict__ m, int64_t n)
+{
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    const double2 x = X[i];
+    X[i] = make_double2(x.x * m[i], x.y * m[i]);
+}
+
+// out += flambda s (scale Re back)
+__global__ __launch_bounds__(256) void k_reg_add(const double2 *__restrict__ back, double scale,
+                                                 const double *__restrict__ s, double flambda,
+                                                 int64_t n, double *__restrict__ out)
+{
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) out[i] += flambda * (back[i].x * scale) * s[i];
+}
+
 unsigned blocks_for(int64_t n, int64_t cap)
 {
     const int64_t b = mtip::ceil_div(n, 256);
@@ -140,6 +213,59 @@ extern "C" int mtip_merge_combine(const double *y_ups, const double *y_reg, cons
     hipLaunchKernelGGL(k_merge_combine, dim3((unsigned)mtip::ceil_div(n, 256)), dim3(256), 0,
                        (hipStream_t)stream, y_ups, y_reg, u, support, M, M_ups, rlambda, flambda,
                        out);
+    MTIP_HIP_CHECK(hipGetLastError());
+    return MTIP_OK;
+}
+
+extern "C" int mtip_merge_reg_embed(const double *u, const double *support, int64_t n, void *w,
+                                    void *stream)
+{
+    MTIP_REQUIRE(n >= 1 && u && support && w, MTIP_ERR_ARG, "mtip_merge_reg_embed: bad argument");
+    hipLaunchKernelGGL(k_reg_embed, dim3((unsigned)mtip::ceil_div(n, 256)), dim3(256), 0,
+                       (hipStream_t)stream, u, support, n, (double2 *)w);
+    MTIP_HIP_CHECK(hipGetLastError());
+    return MTIP_OK;
+}
+
+extern "C" int mtip_merge_reg_mask(void *spectrum, const double *mask, int64_t n, void *stream)
+{
+    MTIP_REQUIRE(n >= 1 && spectrum && mask, MTIP_ERR_ARG, "mtip_merge_reg_mask: bad argument");
+    hipLaunchKernelGGL(k_reg_mask, dim3((unsigned)mtip::ceil_div(n, 256)), dim3(256), 0,
+                       (hipStream_t)stream, (double2 *)spectrum, mask, n);
+    MTIP_HIP_CHECK(hipGetLastError());
+    return MTIP_OK;
+}
+
+extern "C" int mtip_merge_reg_add(const void *back, double scale, const double *support,
+                                  double flambda, int64_t n, double *out, void *stream)
+{
+    MTIP_REQUIRE(n >= 1 && back && support && out, MTIP_ERR_ARG, "mtip_merge_reg_add: bad argument");
+    hipLaunchKernelGGL(k_reg_add, dim3((unsigned)mtip::ceil_div(n, 256)), dim3(256), 0,
+                       (hipStream_t)stream, (const double2 *)back, scale, support, flambda, n, out);
+    MTIP_HIP_CHECK(hipGetLastError());
+    return MTIP_OK;
+}
+
+extern "C" int mtip_half_pack(const void *spectrum, int M, void *half, void *stream)
+{
+    MTIP_REQUIRE(M >= 1 && M % 2 == 1 && M <= 2047, MTIP_ERR_ARG, "mtip_half_pack: M must be odd, at most 2047");
+    MTIP_REQUIRE(spectrum && half, MTIP_ERR_ARG, "mtip_half_pack: null pointer");
+    const dim3 grid((unsigned)mtip::ceil_div((int64_t)M * M, kHalfRows),
+                    (unsigned)mtip::ceil_div(M / 2 + 1, kHalfCols));
+    hipLaunchKernelGGL(k_half_pack, grid, dim3(256), 0, (hipStream_t)stream, (const double2 *)spectrum, M,
+                       (double2 *)half);
+    MTIP_HIP_CHECK(hipGetLastError());
+    return MTIP_OK;
+}
+
+extern "C" int mtip_half_expand(const void *half, int M, void *spectrum, void *stream)
+{
+    MTIP_REQUIRE(M >= 1 && M % 2 == 1 && M <= 2047, MTIP_ERR_ARG, "mtip_half_expand: M must be odd, at most 2047");
+    MTIP_REQUIRE(half && spectrum, MTIP_ERR_ARG, "mtip_half_expand: null pointer");
+    const dim3 grid((unsigned)mtip::ceil_div((int64_t)M * M, kHalfRows),
+                    (unsigned)mtip::ceil_div(M / 2 + 1, kHalfCols));
+    hipLaunchKernelGGL(k_half_expand, grid, dim3(256), 0, (hipStream_t)stream, (const double2 *)half, M,
+                       (double2 *)spectrum);
     MTIP_HIP_CHECK(hipGetLastError());
     return MTIP_OK;
 }
