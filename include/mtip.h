@@ -217,6 +217,14 @@ int mtip_plan_spread_finish(mtip_plan *plan, const double *support, double scale
 int mtip_phase_amplitudes(void *spectrum, const double *amplitudes, int64_t n, void *stream);
 int mtip_phase_update(double *rho, const double *rho_mod, const uint8_t *support, int64_t n,
                       int mode, double beta, double rho_max, void *stream);
+/*
+ * One axis of scipy.ndimage's separable Gaussian filter on FP64 values (outer, n, inner)
+ * (phasing.py:215-216, :258-259; autocorrelation.py:201): out = sum of the 2 radius + 1
+ * host weights times the neighbours along n, radius <= 16; mode 0 reflect, 1 wrap,
+ * 2 constant (zero outside).  in and out differ.
+ */
+int mtip_gauss_axis(const double *in, int64_t outer, int n, int64_t inner, int radius,
+                    const double *weights, int mode, double *out, void *stream);
 
 /* ---------------------------------------------------------------- merge */
 

@@ -4,8 +4,15 @@ default, spinifel/sequential/autocorrelation.py:201), 'constant' (cval 0,
 spinifel/sequential/phasing.py:258-259) and 'wrap' (:215-216).  The kernel
 is scipy's: weights exp(-x^2 / 2 sigma^2) on |x| <= int(truncate sigma + 0.5),
 normalised to sum 1, applied along each axis in turn."""
+import math
+
 import numpy as np
 import torch
+
+from . import _lib, engine
+
+_MODES = {"reflect": 0, "wrap": 1, "constant": 2}
+_MAX_RADIUS = 16        # of mtip_gauss_axis
 
 
 def _index(n, radius, mode, device):
@@ -34,6 +41,9 @@ def gaussian_filter(a, sigma, mode="reflect", truncate=4.0):
     w = np.exp(-0.5 * (x / sigma) ** 2)
     w /= w.sum()
     out = a.to(torch.float64)
+    if out.is_cuda and out.numel() and radius <= _MAX_RADIUS and mode in _MODES \
+            and out.numel() <= 1 << 31:
+        return _filter_axes(out.contiguous(), w, radius, _MODES[mode])
     for ax in range(out.dim()):
         n = out.shape[ax]
         idx, valid = _index(n, radius, mode, out.device)
@@ -47,3 +57,16 @@ def gaussian_filter(a, sigma, mode="reflect", truncate=4.0):
             acc += float(w[t]) * pad.narrow(ax, t, n)
         out = acc
     return out
+
+
+def _filter_axes(a, w, radius, mode):
+    """The loop of ``gaussian_filter``, one kernel an axis (the same products and sums in the same
+    order, so the same bits)."""
+    lib, P, st = _lib.load(), engine._ptr, engine._stream()
+    w = np.ascontiguousarray(w, np.float64)
+    for ax, n in enumerate(a.shape):
+        out = torch.empty_like(a)
+        _lib.check(lib.mtip_gauss_axis(P(a), math.prod(a.shape[:ax]), n, math.prod(a.shape[ax + 1:]),
+                                       radius, w.ctypes.data, mode, P(out), st), "mtip_gauss_axis")
+        a = out
+    return a
