@@ -1458,9 +1458,12 @@ void launch_gemm_topk(const void *S, int64_t lds_b, int64_t N_o, const void *D, 
                       float *edge_ws, hipStream_t st)
 {
     // k_gemm_split addresses a tile's rows with 32-bit buffer offsets (longer
-    // rows, 16 MiB, take the FP32 instructions)
+    // rows, 16 MiB, take the FP32 instructions).  Rows it would leave to them run in
+    // the 128-row kernel where that is the tile (10,000 x 100,000 x 64, 4 best: 2.43
+    // ms, 2.70 in k_gemm_split).
     if constexpr (PREC == MTIP_FP32) {
-        if ((int64_t)BM * std::max(lds_b, ldd_b) < ((int64_t)1 << 31)) {
+        if ((int64_t)BM * std::max(lds_b, ldd_b) < ((int64_t)1 << 31) &&
+            (tile == BM2 || kbytes > 4 * kPlainPix)) {
             launch_split_topk<K>((const float *)S, lds_b / 4, N_o, (const float *)D, ldd_b / 4, N_i,
                                  (int)(kbytes / 4), s2, alpha, tile, part, st);
             return;
