@@ -658,17 +658,19 @@ void launch_slices(const GridView &gv, const double *quats, int64_t N_o, const d
                    const int32_t *orient_order, double gscale, float *out, int64_t ld,
                    uint16_t *obf, double *rs, double *rq, int *bad, hipStream_t st)
 {
-    // Workgroups an orientation: one with many orientations; below 4,096 (five rounds of
-    // the 768 workgroups that fit the chip) 8 trips each, fewer where that leaves less
-    // than two workgroups a place.  One workgroup an orientation leaves CUs idle in the
-    // last round, and with few orientations: 1,000 x 16k points (64 trips) 1,065 us
-    // whole, 918 at 8 trips a part, 953 at 4, 962 at 1; 1,009 x 14k at M = 121 1,553 and
-    // 1,320; 50 x 1,024 points 79 and 55 us.  The row sums then take a pass of their own
-    // over the values (in these figures), which costs 10,000 x 16k points in float32 and
-    // bf16 more than the last round does (the step 12.0 against 11.85 ms).
+    // Workgroups an orientation: 8 trips each, fewer where that leaves less than two
+    // workgroups a place (768 fit the chip).  One workgroup an orientation leaves CUs
+    // idle in the last round, and with few orientations: 1,000 x 16k points (64 trips)
+    // 1,065 us whole, 918 at 8 trips a part, 953 at 4, 962 at 1; 1,009 x 14k at M = 121
+    // 1,553 and 1,320; 4,000 x 16k 3,270 and 3,149; 50 x 1,024 points 79 and 55.  The row
+    // sums then take a pass of their own over the values (in these figures), which with
+    // 256-point tiles and many orientations costs what the split gains (the bf16 step of
+    // 10,000 x 16k points 12.0 ms either way), while smaller tiles still gain (6,000 x
+    // 14k at M = 121 7.11 and 6.79 ms, the fp8 step of 10,007 x 12k 11.72 and 11.49).
     const int64_t trips = mtip::ceil_div(order ? n_order : N_p, 256);
-    const int64_t most =
-        N_o >= 4096 ? trips : std::max<int64_t>(1, std::min<int64_t>(8, trips * N_o / 1536));
+    const int64_t most = N_o >= 4096 && tile != 64 && tile != 128
+                             ? trips
+                             : std::max<int64_t>(1, std::min<int64_t>(8, trips * N_o / 1536));
     const int64_t parts = std::min<int64_t>(mtip::ceil_div(trips, most), 65535);
     const int64_t per = mtip::ceil_div(trips, parts);
     const dim3 wgs((unsigned)N_o, (unsigned)mtip::ceil_div(trips, per));
