@@ -195,6 +195,10 @@ int mtip_plan_spread_points(mtip_plan *plan, const double *x, const double *y, c
  */
 int mtip_plan_spread_finish(mtip_plan *plan, const double *support, double scale, double *out,
                             void *stream);
+/* The same by a plain sum per output in ascending order of the grid points, slower:
+ * for callers to whom the rounding matters (the merge's iteration amplifies it). */
+int mtip_plan_spread_finish_ordered(mtip_plan *plan, const double *support, double scale,
+                                    double *out, void *stream);
 
 /* ---------------------------------------------------------------- phasing */
 
@@ -245,7 +249,8 @@ int mtip_merge_combine(const double *y_ups, const double *y_reg, const double *u
                        double *out, void *stream);
 
 /*
- * Either convolution of the operator without FFTs, 2 <= M <= M_ups <= 320:
+ * Either convolution of the operator without FFTs, 2 <= M <= M_ups <= 320 (other
+ * rounding than the FFTs', which spinifel_amd.merge keeps):
  *   out = scale s . crop(K * pad(s . u)) + coef base,
  * K a real kernel, cyclic on the M_ups grid (M for the regulariser), with spectrum:
  * device complex double (M_ups / 2 + 1, M_ups, M_ups), its forward transform with

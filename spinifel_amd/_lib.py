@@ -47,6 +47,7 @@ _SIGS = {
                                        _i64, _vp, _vp]),
     "mtip_plan_spread_points": (_i32, [_vp, _vp, _vp, _vp, _i64, _vp, _vp, _vp]),
     "mtip_plan_spread_finish": (_i32, [_vp, _vp, _f64, _vp, _vp]),
+    "mtip_plan_spread_finish_ordered": (_i32, [_vp, _vp, _f64, _vp, _vp]),
     "mtip_phase_amplitudes": (_i32, [_vp, _vp, _i64, _vp]),
     "mtip_phase_update": (_i32, [_vp, _vp, _vp, _i64, _i32, _f64, _f64, _vp]),
     "mtip_gauss_axis": (_i32, [_vp, _i64, _i32, _i64, _i32, _vp, _i32, _vp, _vp]),

@@ -10,7 +10,8 @@
 // Only Re f_k is produced: every caller keeps the real part (spinifel's
 // adjoint with use_recip_sym, autocorrelation.py:123-124 and
 // extern/nufft_ext.py:323-324).  For real c the grid b is real, so
-// f~(-k) = conj f~(k): the passes (dft.hip) keep k1 in [0, M/2] only.
+// f~(-k) = conj f~(k): the transforms keep half of one axis only, k1 in
+// [0, M/2] by DFT matrices (dft.hip) and k3 in the plain passes below.
 //
 // b lives on the padded grid of the plan (indices l in [-n/2 - pad,
 // n/2 + pad)), so windows never wrap; the passes add up the padded copies of a
@@ -28,6 +29,8 @@
 #include "nufft_shared.h"
 
 namespace {
+
+constexpr int kAdjOch = 8;         // outputs per thread of a pass in fixed order
 
 __global__ __launch_bounds__(256) void k_zero_f64(double *__restrict__ p, int64_t n)
 {
@@ -347,6 +350,109 @@ __global__ __launch_bounds__(256, 3) void k_spread(GridView gv, double *__restri
     if (nbad && bad) atomicAdd(bad, nbad);
 }
 
+// One separable pass of the transform back to modes, a plain sum per output with the
+// points in ascending order:
+//   out[a][kk][c] = sum_{o < L} in(a, o, c) exp(+2 pi i k l / n),
+//   k = kk + k_lo (kk < NK), l = o - off.
+// MODE 0: real input, complex output.  MODE 1: complex -> complex.
+// MODE 2 (last pass, axis 0, A = 1, c = k2i (h + 1) + k3): writes
+//   out_r[i1][i2][i3] = Re(.) dinv(k1) dinv(k2) dinv(k3) scale support[i]
+// at (k1, k2, k3) and, for k3 > 0, at (-k1, -k2, -k3), where i_d = k_d + M/2.
+//
+// The merge takes these passes, everybody else the DFT matrices (dft.hip).  Its 100
+// iterations, stopped far from convergence, amplify a rounding of 1e-16 in the kernel
+// or the data term to 1e-4 and more of the result, so another order of the sums
+// here changes what every merge returns (by up to 6e-9 where M = 9 and every spread
+// is one workgroup, so that runs give the same bits; at M = 81 two runs of one
+// program already differ by 1e-5 to 9e-4, through the order of the spread's atomics).
+// Bound: a read of the table in LDS per product (M = 41 171 us, DFT matrices 29; M = 81
+// 317 and 68; M = 162 1,945 and 540).
+template <int MODE>
+__global__ __launch_bounds__(256) void k_adj_pass(const double *__restrict__ in_r,
+                                                  const double2 *__restrict__ in_c,
+                                                  double2 *__restrict__ out_c,
+                                                  const double2 *__restrict__ tw, int n, int L,
+                                                  int off, int NK, int k_lo, int64_t A, int64_t C,
+                                                  double *__restrict__ out_r,
+                                                  const double *__restrict__ dinv, int h, int M,
+                                                  const double *__restrict__ support, double scale)
+{
+    extern __shared__ double2 s_tw[];
+    for (int i = threadIdx.x; i < n; i += blockDim.x) s_tw[i] = tw[i];
+    __syncthreads();
+
+    const int nchunk = (NK + kAdjOch - 1) / kAdjOch;
+    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= A * nchunk * C) return;
+    const int64_t c = t % C;
+    const int64_t r = t / C;
+    const int chunk = (int)(r % nchunk);
+    const int64_t a = r / nchunk;
+    const int kk0 = chunk * kAdjOch;
+
+    // phase index (k l) mod n of each output, advanced by k mod n per input
+    const int l0 = ((-off) % n + n) % n;
+    int idx[kAdjOch], step[kAdjOch];
+#pragma unroll
+    for (int j = 0; j < kAdjOch; ++j) {
+        const int k = kk0 + j + k_lo;
+        step[j] = ((k % n) + n) % n;
+        idx[j] = (int)(((int64_t)step[j] * l0) % n);
+    }
+    double acc_re[kAdjOch], acc_im[kAdjOch];
+#pragma unroll
+    for (int j = 0; j < kAdjOch; ++j) acc_re[j] = acc_im[j] = 0.0;
+
+    for (int o = 0; o < L; ++o) {
+        double vr, vi = 0.0;
+        if (MODE == 0) {
+            vr = in_r[a * L + o];
+        } else {
+            const double2 v = in_c[(a * L + o) * C + c];
+            vr = v.x;
+            vi = v.y;
+        }
+#pragma unroll
+        for (int j = 0; j < kAdjOch; ++j) {
+            // tw = exp(-i theta): exp(+i theta) = (tw.x, -tw.y)
+            const double2 e = s_tw[idx[j]];
+            const double cs = e.x, sn = -e.y;
+            if (MODE == 0) {
+                acc_re[j] = fma(vr, cs, acc_re[j]);
+                acc_im[j] = fma(vr, sn, acc_im[j]);
+            } else {
+                acc_re[j] = fma(vr, cs, fma(-vi, sn, acc_re[j]));
+                acc_im[j] = fma(vr, sn, fma(vi, cs, acc_im[j]));
+            }
+            idx[j] += step[j];
+            idx[j] -= idx[j] >= n ? n : 0;
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < kAdjOch; ++j) {
+        const int kk = kk0 + j;
+        if (kk >= NK) break;
+        if (MODE != 2) {
+            out_c[(a * NK + kk) * C + c] = make_double2(acc_re[j], acc_im[j]);
+        } else {
+            const int k1 = kk + k_lo;
+            const int hp1 = h + 1;
+            const int k2 = (int)(c / hp1) - h, k3 = (int)(c % hp1);
+            const double val =
+                acc_re[j] * dinv[k1 + h] * dinv[k2 + h] * dinv[k3 + h] * scale;
+            const int lo = -(M / 2), hi = (M - 1) / 2;
+            if (k1 <= hi && k2 <= hi && k3 <= hi) {
+                const int64_t i = ((int64_t)(k1 - lo) * M + (k2 - lo)) * M + (k3 - lo);
+                out_r[i] = support ? val * support[i] : val;
+            }
+            if (k3 > 0 && -k1 >= lo && -k1 <= hi && -k2 >= lo && -k2 <= hi && -k3 >= lo) {
+                const int64_t i = ((int64_t)(-k1 - lo) * M + (-k2 - lo)) * M + (-k3 - lo);
+                out_r[i] = support ? val * support[i] : val;
+            }
+        }
+    }
+}
+
 template <int W>
 void launch_spread(const GridView &gv, double *acc, int geom, const double *quats, int64_t N_o,
                    const double *q, int64_t N_p, const int32_t *order, int64_t n_order, int tile,
@@ -466,4 +572,40 @@ extern "C" int mtip_plan_spread_finish(mtip_plan *p, const double *support, doub
     MTIP_REQUIRE(std::isfinite(scale), MTIP_ERR_ARG, "mtip_plan_spread_finish: scale not finite");
     DeviceGuard dg(p->device);
     return mtip::modes_from_grid(p, support, scale, out, (hipStream_t)stream);
+}
+
+extern "C" int mtip_plan_spread_finish_ordered(mtip_plan *p, const double *support, double scale,
+                                               double *out, void *stream)
+{
+    MTIP_REQUIRE(p && out, MTIP_ERR_ARG, "mtip_plan_spread_finish_ordered: null argument");
+    MTIP_REQUIRE(p->spread_open, MTIP_ERR_STATE,
+                 "mtip_plan_spread_finish_ordered: mtip_plan_spread_begin not called");
+    MTIP_REQUIRE(std::isfinite(scale), MTIP_ERR_ARG, "mtip_plan_spread_finish_ordered: scale not finite");
+    DeviceGuard dg(p->device);
+    hipStream_t st = (hipStream_t)stream;
+    const int np = p->np, h = p->h, K = p->K, n = p->n;
+    const int nh = h + 1;
+    const size_t shm = n * sizeof(double2);
+    auto nblk = [](int64_t A, int NK, int64_t C) {
+        return (unsigned)mtip::ceil_div(A * ((NK + kAdjOch - 1) / kAdjOch) * C, 256);
+    };
+    // pass 0: axis 2 (l3 -> k3 in [0, h]), real input [l1 l2][l3]
+    int64_t A = (int64_t)np * np, C = 1;
+    hipLaunchKernelGGL(k_adj_pass<0>, dim3(nblk(A, nh, C)), dim3(256), shm, st, p->acc, nullptr,
+                       p->a1, p->tw, n, np, p->off, nh, 0, A, C, nullptr, nullptr, h, p->M,
+                       nullptr, 0.0);
+    // pass 1: axis 1 (l2 -> k2 in [-h, h]), input [l1][l2][k3]
+    A = np;
+    C = nh;
+    hipLaunchKernelGGL(k_adj_pass<1>, dim3(nblk(A, K, C)), dim3(256), shm, st, nullptr, p->a1,
+                       p->a2, p->tw, n, np, p->off, K, -h, A, C, nullptr, nullptr, h, p->M,
+                       nullptr, 0.0);
+    // pass 2: axis 0 (l1 -> k1 in [-h, h]), input [l1][k2 k3], real output
+    A = 1;
+    C = (int64_t)K * nh;
+    hipLaunchKernelGGL(k_adj_pass<2>, dim3(nblk(A, K, C)), dim3(256), shm, st, nullptr, p->a2,
+                       nullptr, p->tw, n, np, p->off, K, -h, A, C, out, p->dinv, h, p->M, support,
+                       scale);
+    MTIP_HIP_CHECK(hipGetLastError());
+    return MTIP_OK;
 }

@@ -302,7 +302,8 @@ __global__ __launch_bounds__(512) void k_grid_axis3(const double2 *__restrict__ 
 
 // ---------------------------------- convolution with a kernel given by its spectrum
 //
-// out = scale s . crop(K * pad(s . u)) + coef base on M^3 values, K cyclic on n^3
+// out = scale s . crop(K * pad(s . u)) + coef base on M^3 values (mtip_merge_conv, for C
+// callers; Merge keeps the FFTs' rounding, see adjoint.hip), K cyclic on n^3
 // points, n >= M, F its spectrum (l1 in [0, n/2], l2, l3).  Axis 1 and 2 forward,
 // then axis 3 forward, the product with F and axis 3 back in one kernel, so the
 // full spectrum of u is never stored, then axis 2 and 1 back.  Value i of an axis

@@ -73,6 +73,17 @@ double es_phi_host(double z, int w, double beta)
     return v > 0.0 ? exp(beta * (sqrt(v) - 1.0)) : 0.0;
 }
 
+// tw[m] = exp(-2 pi i m / n)
+__global__ void k_twiddle(double2 *tw, int n)
+{
+    int m = blockIdx.x * blockDim.x + threadIdx.x;
+    if (m < n) {
+        double s, c;
+        sincospi(2.0 * (double)m / (double)n, &s, &c);
+        tw[m] = make_double2(c, -s);
+    }
+}
+
 // ------------------------------------------------------------ interpolation
 //
 // Lane layout: a group of G lanes (G = 4, 8 or 16 >= w) interpolates one
@@ -745,6 +756,11 @@ extern "C" int mtip_plan_create(int M, double eps, int device, mtip_plan **out)
     if (err == hipSuccess) err = hipMalloc(&p->dinv, p->K * sizeof(double));
     if (err == hipSuccess)
         err = hipMemcpy(p->dinv, dinv.data(), p->K * sizeof(double), hipMemcpyHostToDevice);
+    if (err == hipSuccess) err = hipMalloc(&p->tw, p->n * sizeof(double2));
+    if (err == hipSuccess) {
+        hipLaunchKernelGGL(k_twiddle, dim3((p->n + 255) / 256), dim3(256), 0, 0, p->tw, p->n);
+        err = hipGetLastError();
+    }
     if (err == hipSuccess) err = hipDeviceSynchronize();
     if (err != hipSuccess) {
         std::string msg = std::string("mtip_plan_create: ") + hipGetErrorString(err);
@@ -762,6 +778,7 @@ extern "C" int mtip_plan_destroy(mtip_plan *p)
     DeviceGuard dg(p->device);
     (void)hipFree(p->grid);
     (void)hipFree(p->dinv);
+    (void)hipFree(p->tw);
     (void)hipFree(p->G);
     (void)hipFree(p->acc);
     (void)hipFree(p->a1);

@@ -15,6 +15,7 @@ struct mtip_plan {
     double beta = 0.0, eps = 0.0;
     float *grid = nullptr;        // (np)^3 real fine grid
     double *dinv = nullptr;       // K: 1 / phihat(k)
+    double2 *tw = nullptr;        // n: exp(-2 pi i m / n)
     double2 *G = nullptr;         // trig table and the two half-transformed models (dft.hip)
     bool loaded = false;
     // type-1 (adjoint) state, allocated on first use

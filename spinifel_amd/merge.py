@@ -16,10 +16,8 @@ Where the work runs:
     term at M with the support) -- libmtip's spreading kernel and transform
     passes, positions formed on the fly from the quaternions (no H, K, L
     arrays), the images resident in HBM as FP32;
-  * per iteration, the convolution on the M_ups^3 grid -- libmtip's transforms
-    by DFT matrices, which neither store nor transform the padding (90 us at
-    M = 81, M_ups = 162; an FFT pair with its copies took 220 us) -- and the
-    Fourier regulariser on M^3 -- rocFFT through torch.fft, in FP64, as
+  * the per-iteration FFTs (the convolution on the M_ups^3 grid and the
+    Fourier regulariser on M^3) -- rocFFT through torch.fft, in FP64, as
     real-to-complex transforms: every operand is real and every product
     Hermitian, so irfftn(rfftn(.) * half-spectrum) equals the reference's
     real part of ifftn(fftn(.) * spectrum) (the regulariser's mask is
@@ -170,29 +168,10 @@ def cg_fused(matvec, b, x0, maxiter, tol=1e-5, callback=None):
     return x, info, it
 
 
-class _Convolution:
-    """out = scale s . crop(K * pad(s . u)) + coef base by libmtip's pruned transforms,
-    K given by its spectrum (n / 2 + 1, n, n), with a workspace of its own."""
-
-    def __init__(self, lib, M, n, spectrum, device):
-        self.lib, self.M, self.n, self.spectrum = lib, M, n, spectrum
-        self.work = torch.empty(int(lib.mtip_merge_conv_workspace_size(M, n)) // 8,
-                                dtype=torch.float64, device=device)
-        _lib.check(lib.mtip_merge_conv_prepare(M, n, engine._ptr(self.work), self.work.numel() * 8,
-                                               engine._stream()), "mtip_merge_conv_prepare")
-
-    def __call__(self, u, support, scale, coef, base, out):
-        P = engine._ptr
-        _lib.check(self.lib.mtip_merge_conv(P(u), P(support), P(self.spectrum), self.M, self.n,
-                                            scale, coef, P(base), P(self.work),
-                                            self.work.numel() * 8, P(out), engine._stream()),
-                   "mtip_merge_conv")
-
-
 class _Regulariser:
-    """out += flambda s . irfftn(rfftn(s . u) * mask) on M^3 values.  Odd M: axis by axis
-    on complex transforms -- the values of the real ones bit for bit (odd lengths
-    run as complex ones there too) without their copies between the axes (M = 81: 84
+    """irfftn(rfftn(s . u) * mask) on M^3 values.  Odd M: axis by axis on complex
+    transforms -- the values of the real ones bit for bit (odd lengths run as
+    complex ones there too) without their copies between the axes (M = 81: 84
     -> 60 us)."""
 
     def __init__(self, lib, M, mask):
@@ -203,13 +182,9 @@ class _Regulariser:
             self.full = torch.empty((M,) * 3, dtype=torch.complex128, device=mask.device)
             self.half = torch.empty((M // 2 + 1, M, M), dtype=torch.complex128, device=mask.device)
 
-    def __call__(self, u, support, flambda, out):
+    def _back(self, u, support):
+        """Odd M: M^3 times the values, as the real parts of complex ones."""
         M, n = self.M, self.M ** 3
-        if not self.odd:
-            R = torch.fft.rfftn(u.view(M, M, M) * support)
-            R *= self.mask
-            out.view(M, M, M).addcmul_(torch.fft.irfftn(R, s=(M, M, M)), support, value=flambda)
-            return
         lib, P, st = self.lib, engine._ptr, engine._stream()
         _lib.check(lib.mtip_merge_reg_embed(P(u), P(support), n, P(self.full), st),
                    "mtip_merge_reg_embed")
@@ -219,9 +194,25 @@ class _Regulariser:
         _lib.check(lib.mtip_merge_reg_mask(P(R), P(self.mask), R.numel(), st), "mtip_merge_reg_mask")
         Z = torch.fft.ifftn(R, dim=(1, 2), norm="forward")
         _lib.check(lib.mtip_half_expand(P(Z), M, P(self.full), st), "mtip_half_expand")
-        back = torch.fft.ifft(self.full, dim=2, norm="forward")
-        _lib.check(lib.mtip_merge_reg_add(P(back), 1.0 / n, P(support), flambda, n, P(out), st),
-                   "mtip_merge_reg_add")
+        return torch.fft.ifft(self.full, dim=2, norm="forward")
+
+    def values(self, u, support):
+        M = self.M
+        if self.odd:
+            return (self._back(u, support).real * (1.0 / M ** 3)).contiguous()
+        R = torch.fft.rfftn(u.view(M, M, M) * support)
+        R *= self.mask
+        return torch.fft.irfftn(R, s=(M, M, M)).contiguous()
+
+    def __call__(self, u, support, flambda, out):
+        """out += flambda s . values."""
+        M, n = self.M, self.M ** 3
+        if not self.odd:
+            out.view(M, M, M).addcmul_(self.values(u, support), support, value=flambda)
+            return
+        P = engine._ptr
+        _lib.check(self.lib.mtip_merge_reg_add(P(self._back(u, support)), 1.0 / n, P(support), flambda,
+                                               n, P(out), engine._stream()), "mtip_merge_reg_add")
 
 
 class Merge:
@@ -268,6 +259,7 @@ class Merge:
         self._plan_ups = get_plan(self.M_ups, self.eps, self.device.index or 0)
         # zero-padded operand of the convolution; only [:M]^3 is ever written
         self._ups = torch.zeros((self.M_ups,) * 3, dtype=torch.float64, device=self.device)
+        self._us = torch.empty((self.M,) * 3, dtype=torch.float64, device=self.device)
 
         def callback(xk):
             callback.counter += 1
@@ -338,33 +330,43 @@ class Merge:
         quats = self._quats(orientations)
         (x, y, z), data_pts = self._points(quats)
         ugrid_conv = self._plan_ups.adjoint_points(x, y, z, values=None,
-                                                   out_scale=1.0 / self.M_ups ** 3, spatial=False)
+                                                   out_scale=1.0 / self.M_ups ** 3, spatial=False,
+                                                   ordered=True)
         del x, y, z
-        conv = torch.fft.ifftshift(ugrid_conv) / self.M ** 3
-        del ugrid_conv
-        # the real kernel's spectrum, halved along the first axis
-        F = torch.fft.fftn(torch.fft.rfft(conv, dim=0), dim=(1, 2)).contiguous()
-        del conv
-        M = self.M
+        F_half = torch.fft.rfftn(torch.fft.ifftshift(ugrid_conv)) / self.M ** 3
+
+        lib = _lib.load()
+        P = engine._ptr
         sup = ac_support.contiguous()
-        data = _Convolution(_lib.load(), M, self.M_ups, F, self.device)
-        reg = _Regulariser(_lib.load(), M, self._reg_mask)
+        reg = _Regulariser(lib, self.M, self._reg_mask)
 
         def W_matvec(uvect):
             # the same operator as core_problem_convolution + rlambda u +
-            # flambda fourier_reg.  The regulariser keeps its FFT pair on M^3: with
-            # its weight of 1e3 it decides how rounding carries through the
-            # unconverged iterations, which the data term's rounding does not touch
+            # flambda fourier_reg, with the padding and the recombination in
+            # two kernels around the FFTs.  The iteration, stopped far from
+            # convergence, amplifies rounding of 1e-16 in any of the terms to
+            # 1e-4 and more of the result, so the order of the sums in the
+            # kernel, the data term and here is part of what solve_ac returns:
+            # the convolution stays on the FFTs (220 us, by DFT matrices 90)
+            M, Mu = self.M, self.M_ups
             u = uvect.contiguous()
+            st = engine._stream()
+            _lib.check(lib.mtip_merge_pad(P(u), P(sup), M, Mu, P(self._ups), P(self._us), st),
+                       "mtip_merge_pad")
+            X = torch.fft.rfftn(self._ups)
+            X *= F_half
+            y_ups = torch.fft.irfftn(X, s=(Mu,) * 3).contiguous()
+            y_reg = reg.values(u, sup)
             out = torch.empty(M ** 3, dtype=torch.float64, device=self.device)
-            data(u, sup, 1.0, float(self.rlambda), u, out)
-            reg(u, sup, float(self.flambda), out)
+            _lib.check(lib.mtip_merge_combine(P(y_ups), P(y_reg), P(u), P(sup), M, Mu,
+                                              float(self.rlambda), float(self.flambda), P(out),
+                                              st), "mtip_merge_combine")
             return out
 
         xd, yd, zd, vd = data_pts
         uvect_ADb = self._plan.adjoint_points(xd, yd, zd, values=vd, support=ac_support,
                                               out_scale=1.0 / self.M ** 3,
-                                              spatial=False).reshape(-1)
+                                              spatial=False, ordered=True).reshape(-1)
         d = uvect_ADb + self.rlambda * x0
         return W_matvec, d
 
