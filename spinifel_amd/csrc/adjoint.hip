@@ -485,15 +485,12 @@ extern "C" int mtip_plan_spread_begin(mtip_plan *p, void *stream)
         hipError_t err = hipMalloc(&p->acc, n_acc * sizeof(double));
         if (err == hipSuccess) err = hipMalloc(&p->a1, n_a1 * sizeof(double2));
         if (err == hipSuccess) err = hipMalloc(&p->a2, n_a2 * sizeof(double2));
-        if (err == hipSuccess) err = hipMalloc(&p->at, mtip::modes_table_entries(p) * sizeof(double2));
-        if (err == hipSuccess) err = mtip::modes_table(p, (hipStream_t)stream);
         if (err != hipSuccess) {
             (void)hipFree(p->acc);
             (void)hipFree(p->a1);
             (void)hipFree(p->a2);
-            (void)hipFree(p->at);
             p->acc = nullptr;
-            p->a1 = p->a2 = p->at = nullptr;
+            p->a1 = p->a2 = nullptr;
             return mtip::fail(err == hipErrorOutOfMemory ? MTIP_ERR_NOMEM : MTIP_ERR_HIP,
                               std::string("mtip_plan_spread_begin: ") + hipGetErrorString(err));
         }

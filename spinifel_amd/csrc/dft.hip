@@ -675,18 +675,16 @@ int grid_from_model(mtip_plan *p, const float *ac, hipStream_t st)
 {
     const int h = p->h, n = p->n, nh = h + 1, no = n / 2 + 1;
     const int Cp = pad_to(nh, 4), Op = pad_to(no, 16);
-    const size_t n_t = (size_t)Cp * Op, n_w1 = (size_t)no * p->K * nh, n_w2 = (size_t)no * n * nh;
+    const size_t n_w1 = (size_t)no * p->K * nh, n_w2 = (size_t)no * n * nh;
     if (!p->G) {
-        hipError_t e = hipMalloc(&p->G, (n_t + n_w1 + n_w2) * sizeof(double2));
+        hipError_t e = hipMalloc(&p->G, (n_w1 + n_w2) * sizeof(double2));
         if (e != hipSuccess) {
             p->G = nullptr;
             return fail(e == hipErrorOutOfMemory ? MTIP_ERR_NOMEM : MTIP_ERR_HIP,
                         std::string("mtip_plan_set_model: ") + hipGetErrorString(e));
         }
-        hipLaunchKernelGGL(k_trig_table, dim3((unsigned)ceil_div(n_t, 256)), dim3(256), 0, st, p->G,
-                           nh, Cp, no, Op, n);
     }
-    double2 *T = p->G, *w1 = T + n_t, *w2 = w1 + n_w1;
+    double2 *T = p->gt, *w1 = p->G, *w2 = w1 + n_w1;
     // the staged columns; the padded rows take their place (at most 45 KiB, M = 320)
     const size_t lds = (size_t)Cp * 16 * sizeof(double2);
     const size_t lds3 = std::max((size_t)Cp * 17 * sizeof(double2), (size_t)16 * p->np * sizeof(float));
@@ -710,15 +708,23 @@ int grid_from_model(mtip_plan *p, const float *ac, hipStream_t st)
     return MTIP_OK;
 }
 
+size_t grid_table_entries(const mtip_plan *p)
+{
+    return (size_t)pad_to(p->h + 1, 4) * pad_to(p->n / 2 + 1, 16);
+}
+
 size_t modes_table_entries(const mtip_plan *p)
 {
     return (size_t)pad_to(p->n / 2 + 1, 4) * pad_to(p->h + 1, 16);
 }
 
-hipError_t modes_table(const mtip_plan *p, hipStream_t st)
+hipError_t trig_tables(const mtip_plan *p)
 {
-    hipLaunchKernelGGL(k_trig_table, dim3((unsigned)ceil_div(modes_table_entries(p), 256)), dim3(256), 0, st,
-                       p->at, p->n / 2 + 1, pad_to(p->n / 2 + 1, 4), p->h + 1, pad_to(p->h + 1, 16), p->n);
+    const int nh = p->h + 1, no = p->n / 2 + 1;
+    hipLaunchKernelGGL(k_trig_table, dim3((unsigned)ceil_div(grid_table_entries(p), 256)), dim3(256), 0, 0,
+                       p->gt, nh, pad_to(nh, 4), no, pad_to(no, 16), p->n);
+    hipLaunchKernelGGL(k_trig_table, dim3((unsigned)ceil_div(modes_table_entries(p), 256)), dim3(256), 0, 0,
+                       p->at, no, pad_to(no, 4), nh, pad_to(nh, 16), p->n);
     return hipGetLastError();
 }
 

@@ -756,10 +756,14 @@ extern "C" int mtip_plan_create(int M, double eps, int device, mtip_plan **out)
     if (err == hipSuccess) err = hipMalloc(&p->dinv, p->K * sizeof(double));
     if (err == hipSuccess)
         err = hipMemcpy(p->dinv, dinv.data(), p->K * sizeof(double), hipMemcpyHostToDevice);
+    // the transforms' tables, complete when the plan is handed out: the first call on a
+    // plan may be on any stream, or recorded into a graph
     if (err == hipSuccess) err = hipMalloc(&p->tw, p->n * sizeof(double2));
+    if (err == hipSuccess) err = hipMalloc(&p->gt, mtip::grid_table_entries(p) * sizeof(double2));
+    if (err == hipSuccess) err = hipMalloc(&p->at, mtip::modes_table_entries(p) * sizeof(double2));
     if (err == hipSuccess) {
         hipLaunchKernelGGL(k_twiddle, dim3((p->n + 255) / 256), dim3(256), 0, 0, p->tw, p->n);
-        err = hipGetLastError();
+        err = mtip::trig_tables(p);
     }
     if (err == hipSuccess) err = hipDeviceSynchronize();
     if (err != hipSuccess) {
@@ -779,6 +783,7 @@ extern "C" int mtip_plan_destroy(mtip_plan *p)
     (void)hipFree(p->grid);
     (void)hipFree(p->dinv);
     (void)hipFree(p->tw);
+    (void)hipFree(p->gt);
     (void)hipFree(p->G);
     (void)hipFree(p->acc);
     (void)hipFree(p->a1);

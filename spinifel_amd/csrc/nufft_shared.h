@@ -16,13 +16,14 @@ struct mtip_plan {
     float *grid = nullptr;        // (np)^3 real fine grid
     double *dinv = nullptr;       // K: 1 / phihat(k)
     double2 *tw = nullptr;        // n: exp(-2 pi i m / n)
-    double2 *G = nullptr;         // trig table and the two half-transformed models (dft.hip)
+    double2 *gt = nullptr;        // trig table of the transform to the grid (dft.hip)
+    double2 *at = nullptr;        // trig table of the transform back (dft.hip)
+    double2 *G = nullptr;         // the two half-transformed models (dft.hip)
     bool loaded = false;
     // type-1 (adjoint) state, allocated on first use
     double *acc = nullptr;        // (np)^3 FP64 spreading grid
     double2 *a1 = nullptr;        // np * np * (h + 1)
     double2 *a2 = nullptr;        // np * K * (h + 1)
-    double2 *at = nullptr;        // trig table of the transform back (dft.hip)
     bool spread_open = false;     // mtip_plan_spread_begin called
 };
 
@@ -31,10 +32,13 @@ namespace mtip {
 // Fine grid of a plan from its model (dft.hip).
 int grid_from_model(mtip_plan *p, const float *ac, hipStream_t st);
 
-// Entries and contents of the trig table p->at, and the modes of the spread grid
-// p->acc (dft.hip).
+// Entries of the trig tables p->gt and p->at, and their contents, launched on the null
+// stream (dft.hip).
+size_t grid_table_entries(const mtip_plan *p);
 size_t modes_table_entries(const mtip_plan *p);
-hipError_t modes_table(const mtip_plan *p, hipStream_t st);
+hipError_t trig_tables(const mtip_plan *p);
+
+// Modes of the spread grid p->acc by DFT matrices (dft.hip).
 int modes_from_grid(mtip_plan *p, const double *support, double scale, double *out, hipStream_t st);
 
 }  // namespace mtip
