@@ -570,18 +570,21 @@ __global__ __launch_bounds__(512) void k_gemm_big(const uint8_t *__restrict__ A,
 
 // ---------------------------------------------------------------- FP32 cross term
 //
-// FP32 operands on the bf16 matrix instructions: every FP32 value is the exact
-// sum of three bf16 values (8 + 8 + 8 bits, each the rounding of what the ones
-// before leave), split while a stage goes from registers to LDS.  Of the nine
-// partial products the six of relative size 2^-16 and above are accumulated in
-// FP32; the three left out are below 2^-25 of |a b|, half an FP32 rounding.
+// FP32 operands on the bf16 matrix instructions: an FP32 value is the sum of three
+// bf16 values (8 + 8 + 8 bits, each the rounding of what the ones before leave), split
+// while a stage goes from registers to LDS.  Of the nine partial products the six
+// that can reach 2^-17 of |a b| are accumulated in FP32; the three left out are at most
+// 2^-25, 2^-25 and 2^-34 of it, together one FP32 rounding.
 // The bf16 instructions run 16 times the FP32 ones' rate, so six of them cost
 // 6 / 16 of the FP32 product's time, and a sum takes 6 roundings per 16 pixels
 // instead of 16: the error against 64 bits is 0.6 - 0.9 of the FP32 instructions'
 // (16 to 16,384 pixels, normal, uniform and centred photon data; equal on data
-// of a wide range).  10,000 x 10,000 x 16,384: 26.8 -> 16.2 ms.  A tile whose sums are not all finite (an infinity or a NaN in an
-// operand, a sum beyond FP32) is computed again with the FP32 instructions, so
-// such values rank as they do there.
+// of a wide range).  10,000 x 10,000 x 16,384: 26.8 -> 16.2 ms.
+//
+// A sum that is not finite (an infinity or a NaN in an operand, a sum beyond FP32)
+// is computed again with the FP32 instructions, so such values rank as they do there,
+// and it alone: the other sums of its tile keep theirs, whichever rows and
+// columns share the tile.
 //
 // A workgroup of WM x WN waves owns a tile of 32 NI WM orientations x 64 WN images,
 // each wave NI x 2 blocks of 32 x 32: 256 x 256 in 2 x 4 waves of 128 x 64, 128 x
@@ -650,15 +653,12 @@ __global__ __launch_bounds__(64 * WM * WN) void k_gemm_split(
         s_rowc[i] = r < NA ? (float)(al * al * sumsqA[r]) : 0.0f;
     }
     floatx16 acc[NI][2];
-    auto clear = [&]() __attribute__((always_inline)) {
 #pragma unroll
-        for (int i = 0; i < NI; ++i)
+    for (int i = 0; i < NI; ++i)
 #pragma unroll
-            for (int j = 0; j < 2; ++j)
+        for (int j = 0; j < 2; ++j)
 #pragma unroll
-                for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.0f;
-    };
-    clear();
+            for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.0f;
     typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
     const int rowsA = (int)min((int64_t)TM, NA - a0), rowsB = (int)min((int64_t)TN, NB - b0);
     const __amdgpu_buffer_rsrc_t rsA = __builtin_amdgcn_make_buffer_rsrc(
@@ -787,17 +787,23 @@ __global__ __launch_bounds__(64 * WM * WN) void k_gemm_split(
             __syncthreads();
         }
     }
-    // infinities and NaN: this tile again, plainly
-    bool fine = true;
+    // sums that are not finite, again with the FP32 instructions, 64 columns a wave
+    // in two halves
+    auto lost = [&](float v) __attribute__((always_inline)) { return plain || !(fabsf(v) <= 3.402823466e38f); };
+    constexpr int PK = 32;      // pixels a stage
 #pragma unroll
-    for (int i = 0; i < NI; ++i)
+    for (int j = 0; j < 2; ++j) {
+        bool fine = true;
 #pragma unroll
-        for (int j = 0; j < 2; ++j)
+        for (int i = 0; i < NI; ++i)
 #pragma unroll
-            for (int v = 0; v < 16; ++v) fine &= fabsf(acc[i][j][v]) <= 3.402823466e38f;
-    if (__syncthreads_or(!fine || plain)) {
-        clear();
-        constexpr int PK = 32;      // pixels a stage
+            for (int v = 0; v < 16; ++v) fine &= !lost(acc[i][j][v]);
+        if (!__syncthreads_or(!fine)) continue;
+        floatx16 re[NI];
+#pragma unroll
+        for (int i = 0; i < NI; ++i)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) re[i][v] = 0.0f;
         for (int k0 = 0; k0 < n_pix; k0 += PK) {
             for (int c = tid; c < (TM + TN) * (PK / 4); c += NT) {
                 const int r = c / (PK / 4), col = k0 + 4 * (c % (PK / 4));
@@ -810,22 +816,25 @@ __global__ __launch_bounds__(64 * WM * WN) void k_gemm_split(
             __syncthreads();
             for (int g = 0; g < PK / 8; ++g) {
                 const int off = g * 32 + half * 16;
-                floatx4 av[NI], bv[2];
+                floatx4 av[NI];
 #pragma unroll
                 for (int i = 0; i < NI; ++i)
                     av[i] = *(const floatx4 *)(smem + (wm * 32 * NI + i * 32 + l32) * LDS_STRIDE + off);
-#pragma unroll
-                for (int j = 0; j < 2; ++j)
-                    bv[j] = *(const floatx4 *)(smem + (TM + wn * 64 + j * 32 + l32) * LDS_STRIDE + off);
+                const floatx4 bv = *(const floatx4 *)(smem + (TM + wn * 64 + j * 32 + l32) * LDS_STRIDE + off);
 #pragma unroll
                 for (int t = 0; t < 4; ++t)
 #pragma unroll
                     for (int i = 0; i < NI; ++i)
-#pragma unroll
-                        for (int j = 0; j < 2; ++j)
-                            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(av[i][t], bv[j][t], acc[i][j], 0, 0, 0);
+                        re[i] = __builtin_amdgcn_mfma_f32_32x32x2f32(av[i][t], bv[t], re[i], 0, 0, 0);
             }
             __syncthreads();
+        }
+#pragma unroll
+        for (int i = 0; i < NI; ++i) {
+            // compared anew: the lane masks kept from above would spill
+            asm volatile("" : "+v"(acc[i][j]));
+#pragma unroll
+            for (int v = 0; v < 16; ++v) acc[i][j][v] = lost(acc[i][j][v]) ? re[i][v] : acc[i][j][v];
         }
     }
 

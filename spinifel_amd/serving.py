@@ -26,9 +26,9 @@ that kernel.
 Each request is scaled by its own std ratio (``mtip_segment_scaling_ratio``)
 and every per-image quantity (cross term, top-K keys, FP64 rescore) depends
 only on that image; the GEMM tile height is fixed per model (from its
-orientation count, not the batch size), so the same kernel scores a request
-whatever shares its batch, and a request's result is the same alone and in
-any mix, bitwise.
+orientation count, not the batch size), and the kernels that FP32 batches of
+different sizes take add in one order, so a request's result is the same alone
+and in any mix, bitwise.
 """
 import ctypes
 import threading
