@@ -581,10 +581,12 @@ __global__ __launch_bounds__(512) void k_gemm_big(const uint8_t *__restrict__ A,
 // (16 to 16,384 pixels, normal, uniform and centred photon data; equal on data
 // of a wide range).  10,000 x 10,000 x 16,384: 26.8 -> 16.2 ms.
 //
-// A sum that is not finite (an infinity or a NaN in an operand, a sum beyond FP32)
-// is computed again with the FP32 instructions, so such values rank as they do there,
-// and it alone: the other sums of its tile keep theirs, whichever rows and
-// columns share the tile.
+// The three parts are exact from 2^-110 up to where a bf16 rounds to infinity.  A sum
+// that is not finite (an infinity or a NaN in an operand, a value that rounds to one, a
+// sum beyond FP32) is computed again with the FP32 instructions, so such values rank as
+// they do there, and so are those of a row all of whose values are below 2^-95 (in
+// other rows the loss, 2^-134, does not count beside their values).  They alone: the
+// other sums of a tile keep theirs, whichever rows and columns share the tile.
 //
 // A workgroup of WM x WN waves owns a tile of 32 NI WM orientations x 64 WN images,
 // each wave NI x 2 blocks of 32 x 32: 256 x 256 in 2 x 4 waves of 128 x 64, 128 x
@@ -633,6 +635,7 @@ __global__ __launch_bounds__(64 * WM * WN) void k_gemm_split(
     constexpr int PLAIN = (TM + TN) * LDS_STRIDE;       // a stage of the FP32 instructions
     __shared__ __attribute__((aligned(16))) uint8_t smem[2 * STAGE > PLAIN ? 2 * STAGE : PLAIN];
     __shared__ float s_rowc[TM];
+    __shared__ bool s_small[TM + TN];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave % WM, wn = wave / WM;
@@ -652,13 +655,17 @@ __global__ __launch_bounds__(64 * WM * WN) void k_gemm_split(
         const double al = *alpha;
         s_rowc[i] = r < NA ? (float)(al * al * sumsqA[r]) : 0.0f;
     }
+    // rows of kPlainPix or fewer have no stages: all their sums are left to the FP32
+    // instructions below
+    const bool plain = n_pix <= kPlainPix;
+    const float none = plain ? __builtin_nanf("") : 0.0f;
     floatx16 acc[NI][2];
 #pragma unroll
     for (int i = 0; i < NI; ++i)
 #pragma unroll
         for (int j = 0; j < 2; ++j)
 #pragma unroll
-            for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.0f;
+            for (int v = 0; v < 16; ++v) acc[i][j][v] = none;
     typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
     const int rowsA = (int)min((int64_t)TM, NA - a0), rowsB = (int)min((int64_t)TN, NB - b0);
     const __amdgpu_buffer_rsrc_t rsA = __builtin_amdgcn_make_buffer_rsrc(
@@ -678,9 +685,7 @@ __global__ __launch_bounds__(64 * WM * WN) void k_gemm_split(
         of_a[i] = (wave * 64 + NT * i) >> 1 < TM;
         v_st[i] = ((of_a[i] ? row : row - TM) * (int)(of_a[i] ? lda : ldb) + 8 * h_st) * 4;
     }
-    // loads past the last stage read zeros; rows of kPlainPix or fewer are left to
-    // the FP32 instructions below
-    const bool plain = n_pix <= kPlainPix;
+    // loads past the last stage read zeros
     const int n_stages = plain ? 0 : (n_pix + kSplitK - 1) / kSplitK;
     u32x4 ra[kHalves][2];
     auto load_stage = [&](int st) __attribute__((always_inline)) {
@@ -693,11 +698,13 @@ __global__ __launch_bounds__(64 * WM * WN) void k_gemm_split(
             ra[i][1] = __builtin_amdgcn_raw_buffer_load_b128(rs, o + 16, 0, 0);
         }
     };
-    auto store_half = [&](uint8_t *dst, const u32x4 (&r)[2]) __attribute__((always_inline)) {
+    uint32_t seen[kHalves] = {};        // the bits set in any value of the thread's half rows
+    auto store_half = [&](uint8_t *dst, const u32x4 (&r)[2], uint32_t &bits) __attribute__((always_inline)) {
         u32x4 w[3];
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
             uint32_t p[3];
+            bits |= r[e >> 1][2 * (e & 1)] | r[e >> 1][2 * (e & 1) + 1];
             split_pair(__uint_as_float(r[e >> 1][2 * (e & 1)]), __uint_as_float(r[e >> 1][2 * (e & 1) + 1]), p);
 #pragma unroll
             for (int q = 0; q < 3; ++q) w[q][e] = p[q];
@@ -708,7 +715,7 @@ __global__ __launch_bounds__(64 * WM * WN) void k_gemm_split(
     auto store_stage = [&](int buf) __attribute__((always_inline)) {
 #pragma unroll
         for (int i = 0; i < kHalves; ++i)
-            store_half(smem + buf * STAGE + ((tid + NT * i) >> 1) * kSplitRow + 16 * h_st, ra[i]);
+            store_half(smem + buf * STAGE + ((tid + NT * i) >> 1) * kSplitRow + 16 * h_st, ra[i], seen[i]);
     };
     // blocks of 32 this wave has valid rows and columns for
     const int vi = min(NI, max(0, (rowsA - wm * 32 * NI + 31) >> 5));
@@ -787,9 +794,30 @@ __global__ __launch_bounds__(64 * WM * WN) void k_gemm_split(
             __syncthreads();
         }
     }
+    // rows whose parts may fall below the least bf16: values, and none from 2^-95 on
+    bool small = false;
+#pragma unroll
+    for (int i = 0; i < kHalves; ++i) {
+        const uint32_t row = seen[i] | __shfl_xor(seen[i], 1);
+        const bool is = (row & 0x7fffffffu) != 0 && (row & 0x70000000u) == 0;
+        if (h_st == 0) s_small[(tid + NT * i) >> 1] = is;
+        small |= is;
+    }
+    if (__syncthreads_or(small)) {
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            const bool col = s_small[TM + wn * 64 + j * 32 + l32];
+#pragma unroll
+            for (int i = 0; i < NI; ++i)
+#pragma unroll
+                for (int v = 0; v < 16; ++v)
+                    if (col || s_small[wm * 32 * NI + i * 32 + 8 * (v >> 2) + 4 * half + (v & 3)])
+                        acc[i][j][v] = __builtin_nanf("");
+        }
+    }
     // sums that are not finite, again with the FP32 instructions, 64 columns a wave
     // in two halves
-    auto lost = [&](float v) __attribute__((always_inline)) { return plain || !(fabsf(v) <= 3.402823466e38f); };
+    auto lost = [](float v) __attribute__((always_inline)) { return !(fabsf(v) <= 3.402823466e38f); };
     constexpr int PK = 32;      // pixels a stage
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
