@@ -34,6 +34,18 @@ def _index(n, radius, mode, device):
     return idx, valid
 
 
+def _only_values(t):
+    """Whether a tensor is its values and nothing records or transforms what is done
+    with it: autograd in either direction, vmap, tracing and subclasses take the
+    filter written with torch."""
+    return (type(t) in (torch.Tensor, torch.nn.Parameter)
+            and not (t.requires_grad and torch.is_grad_enabled())
+            and not torch._C._functorch.is_functorch_wrapped_tensor(t)
+            and torch.autograd.forward_ad.unpack_dual(t).tangent is None
+            and torch.utils._python_dispatch._get_current_dispatch_mode() is None
+            and not torch.jit.is_tracing() and not torch.compiler.is_compiling())
+
+
 def gaussian_filter(a, sigma, mode="reflect", truncate=4.0):
     """gaussian_filter(a, sigma, mode=mode, truncate=truncate) of a device tensor."""
     radius = int(truncate * float(sigma) + 0.5)
@@ -42,8 +54,9 @@ def gaussian_filter(a, sigma, mode="reflect", truncate=4.0):
     w /= w.sum()
     out = a.to(torch.float64)
     if out.is_cuda and out.numel() and radius <= _MAX_RADIUS and mode in _MODES \
-            and out.numel() <= 1 << 31:
-        return _filter_axes(out.contiguous(), w, radius, _MODES[mode])
+            and out.numel() <= 1 << 31 and _only_values(out):
+        with torch.cuda.device(out.device):
+            return _filter_axes(out.resolve_neg().contiguous(), w, radius, _MODES[mode])
     for ax in range(out.dim()):
         n = out.shape[ax]
         idx, valid = _index(n, radius, mode, out.device)
