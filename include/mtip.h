@@ -224,8 +224,8 @@ int mtip_phase_update(double *rho, const double *rho_mod, const uint8_t *support
 /*
  * One axis of scipy.ndimage's separable Gaussian filter on FP64 values (outer, n, inner)
  * (phasing.py:215-216, :258-259; autocorrelation.py:201): out = sum of the 2 radius + 1
- * host weights times the neighbours along n, radius <= 16; mode 0 reflect, 1 wrap,
- * 2 constant (zero outside).  in and out differ.
+ * host weights times the neighbours along n < 2^30, radius <= 16; mode 0 reflect, 1 wrap,
+ * 2 constant (zero outside).  in and out differ.  About 2^32 values at most.
  */
 int mtip_gauss_axis(const double *in, int64_t outer, int n, int64_t inner, int radius,
                     const double *weights, int mode, double *out, void *stream);

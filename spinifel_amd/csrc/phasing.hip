@@ -134,12 +134,16 @@ extern "C" int mtip_gauss_axis(const double *in, int64_t outer, int n, int64_t i
                                const double *weights, int mode, double *out, void *stream)
 {
     MTIP_REQUIRE(outer >= 0 && n >= 1 && inner >= 0, MTIP_ERR_ARG, "mtip_gauss_axis: bad sizes");
+    // positions are ints, reflected modulo 2 n
+    MTIP_REQUIRE(n < 1 << 30, MTIP_ERR_ARG, "mtip_gauss_axis: n must be below 2^30");
     MTIP_REQUIRE(radius >= 0 && radius <= kGaussRadius, MTIP_ERR_ARG, "mtip_gauss_axis: radius must be 0 to 16");
     MTIP_REQUIRE(mode >= 0 && mode <= 2, MTIP_ERR_ARG, "mtip_gauss_axis: mode must be 0, 1 or 2");
-    const int64_t total = outer * n * inner;
-    if (total == 0) return MTIP_OK;
+    if (outer == 0 || inner == 0) return MTIP_OK;
     MTIP_REQUIRE(in && weights && out && in != out, MTIP_ERR_ARG, "mtip_gauss_axis: null or equal pointers");
-    MTIP_REQUIRE(mtip::ceil_div(total, 256) <= 0xffffff, MTIP_ERR_ARG, "mtip_gauss_axis: too many values");
+    constexpr int64_t most = 256 * (int64_t)0xffffff;
+    MTIP_REQUIRE(inner <= most / n && outer <= most / (n * inner), MTIP_ERR_ARG,
+                 "mtip_gauss_axis: too many values");
+    const int64_t total = outer * n * inner;
     GaussTaps taps;
     for (int t = 0; t < 2 * kGaussRadius + 1; ++t) taps.w[t] = t <= 2 * radius ? weights[t] : 0.0;
     hipLaunchKernelGGL(k_gauss_axis, dim3((unsigned)mtip::ceil_div(total, 256)), dim3(256), 0,

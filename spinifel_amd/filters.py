@@ -54,7 +54,7 @@ def gaussian_filter(a, sigma, mode="reflect", truncate=4.0):
     w /= w.sum()
     out = a.to(torch.float64)
     if out.is_cuda and out.numel() and radius <= _MAX_RADIUS and mode in _MODES \
-            and out.numel() <= 1 << 31 and _only_values(out):
+            and out.numel() < 1 << 30 and _only_values(out):
         with torch.cuda.device(out.device):
             return _filter_axes(out.resolve_neg().contiguous(), w, radius, _MODES[mode])
     for ax in range(out.dim()):
