@@ -18,6 +18,8 @@
 // through LDS).  Within each 64-element chunk of pixels, lane half h feeds
 // elements [32 h, 32 h + 32) in four MFMA steps, for both operands alike,
 // so every pixel meets itself.
+#include <algorithm>
+
 #include "mtip_internal.h"
 
 namespace {
@@ -419,36 +421,36 @@ __global__ __launch_bounds__(256) void k_merge_distinct(const int32_t *__restric
                                                         float *__restrict__ out_val)
 {
     const int lane = threadIdx.x & 63;
-    const int64_t i = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (i >= N_i) return;
-    uint64_t top[KO];
+    for (int64_t i = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6); i < N_i; i += (int64_t)gridDim.x * 4) {
+        uint64_t top[KO];
 #pragma unroll
-    for (int r = 0; r < KO; ++r) top[r] = KEY_NONE;
-    for (int j = lane; j < n_in; j += 64) {
-        const int32_t id = in_idx[i * n_in + j];
-        if (id < 0) continue;
-        const uint64_t key = mtip::make_key(in_val[i * n_in + j], (uint32_t)id);
-        bool dup = false;
+        for (int r = 0; r < KO; ++r) top[r] = KEY_NONE;
+        for (int j = lane; j < n_in; j += 64) {
+            const int32_t id = in_idx[i * n_in + j];
+            if (id < 0) continue;
+            const uint64_t key = mtip::make_key(in_val[i * n_in + j], (uint32_t)id);
+            bool dup = false;
 #pragma unroll
-        for (int r = 0; r < KO; ++r) dup |= (top[r] == key);
-        if (!dup) mtip::topk_insert<KO>(top, key);
-    }
+            for (int r = 0; r < KO; ++r) dup |= (top[r] == key);
+            if (!dup) mtip::topk_insert<KO>(top, key);
+        }
 #pragma unroll 1
-    for (int r = 0; r < KO; ++r) {
-        uint64_t m = top[0];
-        for (int d = 32; d >= 1; d >>= 1) {
-            const uint64_t o = mtip::shfl_xor_u64(m, d);
-            m = o < m ? o : m;
-        }
-        if (top[0] == m) {
+        for (int r = 0; r < KO; ++r) {
+            uint64_t m = top[0];
+            for (int d = 32; d >= 1; d >>= 1) {
+                const uint64_t o = mtip::shfl_xor_u64(m, d);
+                m = o < m ? o : m;
+            }
+            if (top[0] == m) {
 #pragma unroll
-            for (int e = 0; e + 1 < KO; ++e) top[e] = top[e + 1];
-            top[KO - 1] = KEY_NONE;
-        }
-        if (lane == 0) {
-            const bool ok = m != KEY_NONE;
-            out_idx[i * KO + r] = ok ? (int32_t)(uint32_t)m : -1;
-            out_val[i * KO + r] = ok ? mtip::ordered_to_float((uint32_t)(m >> 32)) : __builtin_inff();
+                for (int e = 0; e + 1 < KO; ++e) top[e] = top[e + 1];
+                top[KO - 1] = KEY_NONE;
+            }
+            if (lane == 0) {
+                const bool ok = m != KEY_NONE;
+                out_idx[i * KO + r] = ok ? (int32_t)(uint32_t)m : -1;
+                out_val[i * KO + r] = ok ? mtip::ordered_to_float((uint32_t)(m >> 32)) : __builtin_inff();
+            }
         }
     }
 }
@@ -695,7 +697,8 @@ extern "C" int mtip_merge_distinct(const int32_t *in_idx, const float *in_val, i
     MTIP_REQUIRE(in_idx && in_val && out_idx && out_val, MTIP_ERR_ARG,
                  "mtip_merge_distinct: null pointer");
     hipStream_t st = (hipStream_t)stream;
-    const dim3 grid((unsigned)mtip::ceil_div(N_i, 4));
+    // a launch takes at most 2^32 threads: waves of larger calls take several images
+    const dim3 grid((unsigned)std::min<int64_t>(mtip::ceil_div(N_i, 4), 1 << 22));
     switch (K_out) {
     case 1: hipLaunchKernelGGL(k_merge_distinct<1>, grid, dim3(256), 0, st, in_idx, in_val, N_i, n_in, out_idx, out_val); break;
     case 2: hipLaunchKernelGGL(k_merge_distinct<2>, grid, dim3(256), 0, st, in_idx, in_val, N_i, n_in, out_idx, out_val); break;
