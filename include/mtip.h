@@ -268,7 +268,7 @@ int mtip_merge_conv(const double *u, const double *support, const void *spectrum
 /*
  * The regulariser's elementwise work between complex transforms of n values (a
  * complex double each): w = (s u, 0); spectrum *= mask (real);
- * out += flambda s (scale Re back).
+ * out += flambda s (scale Re back).  About 2^32 values at most.
  * mtip_half_pack / mtip_half_expand: the half spectrum of M^3 real values, M odd,
  * between spectrum (M, M, M), third axis transformed, and half (M / 2 + 1, M, M), third
  * axis first; expand fills the other half with the conjugates along that axis.

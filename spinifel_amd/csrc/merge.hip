@@ -183,6 +183,9 @@ __global__ __launch_bounds__(256) void k_reg_add(const double2 *__restrict__ bac
     if (i < n) out[i] += flambda * (back[i].x * scale) * s[i];
 }
 
+// of a launch with a thread a value: it takes fewer than 2^32 threads
+constexpr int64_t kMostValues = 256 * (int64_t)0xffffff;
+
 unsigned blocks_for(int64_t n, int64_t cap)
 {
     const int64_t b = mtip::ceil_div(n, 256);
@@ -221,6 +224,7 @@ extern "C" int mtip_merge_reg_embed(const double *u, const double *support, int6
                                     void *stream)
 {
     MTIP_REQUIRE(n >= 1 && u && support && w, MTIP_ERR_ARG, "mtip_merge_reg_embed: bad argument");
+    MTIP_REQUIRE(n <= kMostValues, MTIP_ERR_ARG, "mtip_merge_reg_embed: too many values");
     hipLaunchKernelGGL(k_reg_embed, dim3((unsigned)mtip::ceil_div(n, 256)), dim3(256), 0,
                        (hipStream_t)stream, u, support, n, (double2 *)w);
     MTIP_HIP_CHECK(hipGetLastError());
@@ -230,6 +234,7 @@ extern "C" int mtip_merge_reg_embed(const double *u, const double *support, int6
 extern "C" int mtip_merge_reg_mask(void *spectrum, const double *mask, int64_t n, void *stream)
 {
     MTIP_REQUIRE(n >= 1 && spectrum && mask, MTIP_ERR_ARG, "mtip_merge_reg_mask: bad argument");
+    MTIP_REQUIRE(n <= kMostValues, MTIP_ERR_ARG, "mtip_merge_reg_mask: too many values");
     hipLaunchKernelGGL(k_reg_mask, dim3((unsigned)mtip::ceil_div(n, 256)), dim3(256), 0,
                        (hipStream_t)stream, (double2 *)spectrum, mask, n);
     MTIP_HIP_CHECK(hipGetLastError());
@@ -240,6 +245,7 @@ extern "C" int mtip_merge_reg_add(const void *back, double scale, const double *
                                   double flambda, int64_t n, double *out, void *stream)
 {
     MTIP_REQUIRE(n >= 1 && back && support && out, MTIP_ERR_ARG, "mtip_merge_reg_add: bad argument");
+    MTIP_REQUIRE(n <= kMostValues, MTIP_ERR_ARG, "mtip_merge_reg_add: too many values");
     hipLaunchKernelGGL(k_reg_add, dim3((unsigned)mtip::ceil_div(n, 256)), dim3(256), 0,
                        (hipStream_t)stream, (const double2 *)back, scale, support, flambda, n, out);
     MTIP_HIP_CHECK(hipGetLastError());
