@@ -56,7 +56,9 @@ def gaussian_filter(a, sigma, mode="reflect", truncate=4.0):
     if out.is_cuda and out.numel() and radius <= _MAX_RADIUS and mode in _MODES \
             and out.numel() < 1 << 30 and _only_values(out):
         with torch.cuda.device(out.device):
-            return _filter_axes(out.resolve_neg().contiguous(), w, radius, _MODES[mode])
+            r = _filter_axes(out.resolve_neg().contiguous(), w, radius, _MODES[mode])
+            # the layout that the loop's zeros_like gives the result of a dense view
+            return r if out.is_contiguous() else torch.empty_like(out).copy_(r)
     for ax in range(out.dim()):
         n = out.shape[ax]
         idx, valid = _index(n, radius, mode, out.device)
