@@ -53,7 +53,7 @@ def gaussian_filter(a, sigma, mode="reflect", truncate=4.0):
     w = np.exp(-0.5 * (x / sigma) ** 2)
     w /= w.sum()
     out = a.to(torch.float64)
-    if out.is_cuda and out.numel() and radius <= _MAX_RADIUS and mode in _MODES \
+    if out.is_cuda and out.numel() and 0 <= radius <= _MAX_RADIUS and mode in _MODES \
             and out.numel() < 1 << 30 and _only_values(out):
         with torch.cuda.device(out.device):
             r = _filter_axes(out.resolve_neg().contiguous(), w, radius, _MODES[mode])

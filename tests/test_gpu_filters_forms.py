@@ -31,3 +31,11 @@ def test_result_has_the_layout_of_its_input(a, view, mode):
     assert got.stride() == like.stride()
     # products and sums of the same values in the same order
     assert torch.equal(got.cpu(), want)
+
+
+@pytest.mark.parametrize("sigma,truncate", [(-1.0, 4.0), (1.0, -4.0), (-0.1, 4.0), (4.1, 4.0), (4.2, 4.0)])
+def test_radii_at_the_ends_of_the_kernels_range(a, sigma, truncate):
+    """Below zero the filter is an empty sum; 16 is the kernel's largest, 17 the first beyond."""
+    import torch
+    got, want = _both(a, sigma, "reflect", truncate)
+    assert torch.equal(got.cpu(), want)
