@@ -548,10 +548,12 @@ extern "C" int mtip_group_by_winner(const int32_t *winners, int64_t win_stride, 
     if (N_e > 0)
         hipLaunchKernelGGL(k_count, dim3((unsigned)mtip::ceil_div(N_e, 256)), dim3(256), 0, st,
                            winners, win_stride, (int64_t)n_win, N_e, n_groups, w.counts, w.bad);
-    // the workgroups' sums go where the tasks will be written (k_tasks runs last)
+    // the workgroups' sums go where the tasks will be written (k_tasks runs last); the
+    // first workgroup reads none, so one alone needs no pass for them (5 us a call)
     const unsigned n_scan = (unsigned)mtip::ceil_div(n_groups, kScanPer);
-    hipLaunchKernelGGL(k_scan_sums, dim3(n_scan), dim3(kScanPer), 0, st, w.counts, n_groups,
-                       (int2 *)w.tasks);
+    if (n_scan > 1)
+        hipLaunchKernelGGL(k_scan_sums, dim3(n_scan), dim3(kScanPer), 0, st, w.counts, n_groups,
+                           (int2 *)w.tasks);
     hipLaunchKernelGGL(k_scan_apply, dim3(n_scan), dim3(kScanPer), 0, st, w.counts, n_groups,
                        (const int2 *)w.tasks, w.img_off, w.cursor, w.task_off, w.n_tasks);
     if (N_e > 0)
