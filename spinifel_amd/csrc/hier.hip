@@ -19,6 +19,7 @@
 // elements [32 h, 32 h + 32) in four MFMA steps, for both operands alike,
 // so every pixel meets itself.
 #include <algorithm>
+#include <type_traits>
 
 #include "mtip_internal.h"
 
@@ -408,24 +409,26 @@ __global__ __launch_bounds__(256) void k_group_topk(
 }
 
 // Per image: the K_out smallest distinct keys among its n_in candidate
-// (index, value) pairs (T entries x K each, index -1 = none).  One wave per image:
-// each lane keeps the smallest distinct keys of every 64th pair, then the wave
-// takes its minimum K_out times, every lane that holds it dropping it.  (A thread
-// per image left 12,000 images to 48 workgroups reading 512 pairs one by one: 280
-// us; a wave takes 32.)
-template <int KO>
+// (index, value) pairs (T entries x K each, index -1 = none).  G lanes per image: each
+// keeps the smallest distinct keys of every G-th pair, then the group takes its
+// minimum K_out times, every lane that holds it dropping it.  One lane an image reads its
+// pairs one by one, 64 spend K_out rounds of a wave on it whatever n_in: K_out = 8, 12,345
+// images of 512 pairs 270 us with 1 lane, 49 with 8, 27 with 64; 1,000,000 of 64 pairs
+// 2,190, 207 and 966; of 16 pairs 290, 61 with 4 lanes, 95 and 959.
+template <int KO, int G>
 __global__ __launch_bounds__(256) void k_merge_distinct(const int32_t *__restrict__ in_idx,
                                                         const float *__restrict__ in_val,
                                                         int64_t N_i, int n_in,
                                                         int32_t *__restrict__ out_idx,
                                                         float *__restrict__ out_val)
 {
-    const int lane = threadIdx.x & 63;
-    for (int64_t i = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6); i < N_i; i += (int64_t)gridDim.x * 4) {
+    constexpr int IMAGES = 256 / G;
+    const int lane = threadIdx.x % G;
+    for (int64_t i = (int64_t)blockIdx.x * IMAGES + threadIdx.x / G; i < N_i; i += (int64_t)gridDim.x * IMAGES) {
         uint64_t top[KO];
 #pragma unroll
         for (int r = 0; r < KO; ++r) top[r] = KEY_NONE;
-        for (int j = lane; j < n_in; j += 64) {
+        for (int j = lane; j < n_in; j += G) {
             const int32_t id = in_idx[i * n_in + j];
             if (id < 0) continue;
             const uint64_t key = mtip::make_key(in_val[i * n_in + j], (uint32_t)id);
@@ -434,10 +437,20 @@ __global__ __launch_bounds__(256) void k_merge_distinct(const int32_t *__restric
             for (int r = 0; r < KO; ++r) dup |= (top[r] == key);
             if (!dup) mtip::topk_insert<KO>(top, key);
         }
+        auto put = [&](int r, uint64_t m) __attribute__((always_inline)) {
+            const bool ok = m != KEY_NONE;
+            out_idx[i * KO + r] = ok ? (int32_t)(uint32_t)m : -1;
+            out_val[i * KO + r] = ok ? mtip::ordered_to_float((uint32_t)(m >> 32)) : __builtin_inff();
+        };
+        if constexpr (G == 1) {
+#pragma unroll
+            for (int r = 0; r < KO; ++r) put(r, top[r]);
+            continue;
+        }
 #pragma unroll 1
         for (int r = 0; r < KO; ++r) {
             uint64_t m = top[0];
-            for (int d = 32; d >= 1; d >>= 1) {
+            for (int d = G / 2; d >= 1; d >>= 1) {
                 const uint64_t o = mtip::shfl_xor_u64(m, d);
                 m = o < m ? o : m;
             }
@@ -446,11 +459,7 @@ __global__ __launch_bounds__(256) void k_merge_distinct(const int32_t *__restric
                 for (int e = 0; e + 1 < KO; ++e) top[e] = top[e + 1];
                 top[KO - 1] = KEY_NONE;
             }
-            if (lane == 0) {
-                const bool ok = m != KEY_NONE;
-                out_idx[i * KO + r] = ok ? (int32_t)(uint32_t)m : -1;
-                out_val[i * KO + r] = ok ? mtip::ordered_to_float((uint32_t)(m >> 32)) : __builtin_inff();
-            }
+            if (lane == 0) put(r, m);
         }
     }
 }
@@ -699,13 +708,24 @@ extern "C" int mtip_merge_distinct(const int32_t *in_idx, const float *in_val, i
     MTIP_REQUIRE(in_idx && in_val && out_idx && out_val, MTIP_ERR_ARG,
                  "mtip_merge_distinct: null pointer");
     hipStream_t st = (hipStream_t)stream;
-    // a launch takes at most 2^32 threads: waves of larger calls take several images
-    const dim3 grid((unsigned)std::min<int64_t>(mtip::ceil_div(N_i, 4), 1 << 22));
+    // a launch takes at most 2^32 threads: groups of larger calls take several images
+    auto launch = [&](auto ko, auto lanes) {
+        constexpr int KO = decltype(ko)::value, G = decltype(lanes)::value;
+        const dim3 grid((unsigned)std::min<int64_t>(mtip::ceil_div(N_i, 256 / G), 1 << 22));
+        hipLaunchKernelGGL((k_merge_distinct<KO, G>), grid, dim3(256), 0, st, in_idx, in_val, N_i, n_in, out_idx,
+                           out_val);
+    };
+    auto by_lanes = [&](auto ko) {
+        if (n_in <= 8) launch(ko, std::integral_constant<int, 1>{});
+        else if (n_in <= 16) launch(ko, std::integral_constant<int, 4>{});
+        else if (n_in <= 64) launch(ko, std::integral_constant<int, 8>{});
+        else launch(ko, std::integral_constant<int, 64>{});
+    };
     switch (K_out) {
-    case 1: hipLaunchKernelGGL(k_merge_distinct<1>, grid, dim3(256), 0, st, in_idx, in_val, N_i, n_in, out_idx, out_val); break;
-    case 2: hipLaunchKernelGGL(k_merge_distinct<2>, grid, dim3(256), 0, st, in_idx, in_val, N_i, n_in, out_idx, out_val); break;
-    case 4: hipLaunchKernelGGL(k_merge_distinct<4>, grid, dim3(256), 0, st, in_idx, in_val, N_i, n_in, out_idx, out_val); break;
-    default: hipLaunchKernelGGL(k_merge_distinct<8>, grid, dim3(256), 0, st, in_idx, in_val, N_i, n_in, out_idx, out_val); break;
+    case 1: by_lanes(std::integral_constant<int, 1>{}); break;
+    case 2: by_lanes(std::integral_constant<int, 2>{}); break;
+    case 4: by_lanes(std::integral_constant<int, 4>{}); break;
+    default: by_lanes(std::integral_constant<int, 8>{}); break;
     }
     MTIP_HIP_CHECK(hipGetLastError());
     return MTIP_OK;

@@ -47,3 +47,35 @@ def test_candidates_against_numpy(n_in, K):
         best = sorted({(float(v), int(k)) for k, v in zip(a, b) if k >= 0})[:K]
         best += [(np.inf, -1)] * (K - len(best))
         assert [(float(v), int(k)) for k, v in zip(x, y)] == best
+
+
+# the lanes an image has change after 8, 16 and 64 candidates
+@pytest.mark.parametrize("n_in", [2, 7, 8, 9, 15, 16, 17, 31, 33])
+@pytest.mark.parametrize("K", [1, 2, 4, 8])
+@pytest.mark.parametrize("N", [1, 65, 1000])
+def test_lanes_an_image(n_in, K, N):
+    import torch
+    rng = np.random.default_rng(n_in * K + N)
+    idx = rng.integers(-1, 12, (N, n_in)).astype(np.int32)
+    val = (rng.integers(0, 6, 12)[idx] - 0.5 * (idx % 3)).astype(np.float32)
+    oi, ov = [t.cpu().numpy() for t in _merge(torch.as_tensor(idx).cuda(), torch.as_tensor(val).cuda(), K)]
+    for a, b, x, y in zip(idx, val, oi, ov):
+        best = sorted({(float(v), int(k)) for k, v in zip(a, b) if k >= 0})[:K]
+        best += [(np.inf, -1)] * (K - len(best))
+        assert [(float(v), int(k)) for k, v in zip(x, y)] == best
+
+
+def test_more_images_than_waves_of_64_lanes():
+    """2^22 workgroups of four images: images past 2^24 are second ones of their waves."""
+    import torch
+    n, n_in = (1 << 24) + 5, 65
+    print(f"case: {n} images of {n_in}", flush=True)
+    idx = torch.full((n, n_in), -1, dtype=torch.int32, device="cuda")
+    val = torch.zeros((n, n_in), device="cuda")
+    i = torch.arange(n, dtype=torch.int32, device="cuda")
+    idx[:, 3], val[:, 3] = i, (i % 7).float()
+    idx[:, 64], val[:, 64] = i + 1, (i % 5).float()
+    oi, ov = _merge(idx, val, 1)
+    first = val[:, 3] <= val[:, 64]
+    assert torch.equal(oi[:, 0], torch.where(first, i, i + 1))
+    assert torch.equal(ov[:, 0], torch.minimum(val[:, 3], val[:, 64]))
