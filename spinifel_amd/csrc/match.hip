@@ -1465,6 +1465,11 @@ size_t edge_bytes(int64_t N_o, int64_t N_i)
 // other what four do one after the other: split, LDS round trip, products
 // (2,000 x 500 x 1,024 95 -> 78 us, 1,000 x 1,000 x 5,328 370 -> 264 us, 3,000 x 300
 // x 16,384 1,010 -> 750 us; at 4,000 x 2,000 x 16,384, 512 tiles, 1,500 -> 1,590).
+// Short rows leave most of the time to the top-K, which more waves share: eight a
+// 128 x 128 tile win up to about 48 K values a row against the 256 x 256 tiles (6,000 x
+// 3,000 x 128, K = 8: 134 -> 89 us; 5,000 x 2,500, K = 8: 99 -> 93 at 256 values, 113 both at
+// 384; K = 4: 56 both at 192) and about 128 K against four waves (4,000 x 2,000 x
+// 1,024, K = 8: 180 -> 127 us; x 512, K = 4: 65 -> 64, x 1,024: 109 -> 112).
 template <int K>
 void launch_split_topk(const float *S, int64_t lds, int64_t N_o, const float *D, int64_t ldd,
                        int64_t N_i, int n_pix, const double *s2, const double *alpha, int tile,
@@ -1479,9 +1484,10 @@ void launch_split_topk(const float *S, int64_t lds, int64_t N_o, const float *D,
                        TB, WA, WB, n_key, part)
     if (tile == BM2)
         MTIP_SPLIT(4, 2, 4, false, p.nwa * p.nwb + p.n_thin, p.nta, p.ntb, p.nwa, p.nwb);
-    else if (p.nta * p.ntb >= 192 && (int64_t)BM2 * std::max(lds, ldd) * 4 < ((int64_t)1 << 31))
+    else if (n_pix > 48 * K && p.nta * p.ntb >= 192 &&
+             (int64_t)BM2 * std::max(lds, ldd) * 4 < ((int64_t)1 << 31))
         MTIP_SPLIT(4, 2, 4, true, p.nwa * p.nwb + p.n_thin, p.nta, p.ntb, p.nwa, p.nwb);
-    else if (nta * ntb <= 256)
+    else if (n_pix <= 128 * K || nta * ntb <= 256)
         MTIP_SPLIT(1, 4, 2, false, nta * ntb, nta, ntb, nta, ntb);
     else
         MTIP_SPLIT(2, 2, 2, false, nta * ntb, nta, ntb, nta, ntb);
