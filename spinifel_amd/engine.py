@@ -190,11 +190,22 @@ def auto_tiling(plan, det_shape):
     many pixels at 0.9 Nyquist -- and 8 x 8 blocks beyond (measured: 2,000
     orientations of 32 x 32 pixels, n = 90: 264 us for 8 x 8, 316 for 16 x 16;
     1,000 of 128 x 128, n = 162: 1,088 and 972; 1,009 of 111 x 128, n = 250:
-    1,202 and 1,720).  The autotuner (spinifel_amd.autotune) picks by timing."""
+    1,202 and 1,720).  Kernels narrower than 6 points read less where a box does
+    not fit and gain less by the smaller one: up to 4 points 16 x 16 wins on
+    every grid up to 200 points (2,000 of 32 x 32, n = 90, 4 points: 159 us for
+    8 x 8, 123 for 16 x 16; of 64 x 64, n = 180: 522 and 507), at 5 points up to 100
+    or twice the edge (n = 90: 183 and 168; 90 x 90, n = 162: 1,000 and 790; 64 x
+    64, n = 162: 564 and 636).  The autotuner (spinifel_amd.autotune) picks by timing."""
     if len(tuple(det_shape)) < 2:
         return None
     edge = math.sqrt(math.prod(int(d) for d in det_shape))
-    return tiling(det_shape, (16, 16) if plan.n_fine <= 1.6 * edge else (8, 8))
+    width = getattr(plan, "width", 7)
+    most = 1.6 * edge
+    if width <= 4:
+        most = max(most, 200)
+    elif width == 5:
+        most = max(most, 100, min(200, 2 * edge))
+    return tiling(det_shape, (16, 16) if plan.n_fine <= most else (8, 8))
 
 
 def auto_spread_tiling(plan, det_shape):
