@@ -678,10 +678,15 @@ void launch_slices(const GridView &gv, const double *quats, int64_t N_o, const d
     // 256-point tiles and many orientations costs what the split gains (the bf16 step of
     // 10,000 x 16k points 12.0 ms either way), while smaller tiles still gain (6,000 x
     // 14k at M = 121 7.11 and 6.79 ms, the fp8 step of 10,007 x 12k 11.72 and 11.49).
+    // A narrow kernel's trips are short beside that pass and its launch, which cost more
+    // than few trips gain (one orientation of 1,024 points: 2 points wide 18.5 us whole
+    // and 22.2 split, 4 wide 21.0 and 22.1, 5 wide 23.6 and 22.2, 7 wide 38.9 and 22.2)
+    // and as much as it gains from about 2,000 orientations on (4 wide, 3,000 x 4,096
+    // points: 427 and 446).
     const int64_t trips = mtip::ceil_div(order ? n_order : N_p, 256);
-    const int64_t most = N_o >= 4096 && tile != 64 && tile != 128
-                             ? trips
-                             : std::max<int64_t>(1, std::min<int64_t>(8, trips * N_o / 1536));
+    const bool whole = trips * W < 14 || (N_o >= (W <= 4 ? 2048 : 4096) && tile != 64 && tile != 128);
+    const int64_t most = whole ? std::max<int64_t>(1, trips)
+                               : std::max<int64_t>(1, std::min<int64_t>(8, trips * N_o / 1536));
     const int64_t parts = std::min<int64_t>(mtip::ceil_div(trips, most), 65535);
     const int64_t per = mtip::ceil_div(trips, parts);
     const dim3 wgs((unsigned)N_o, (unsigned)mtip::ceil_div(trips, per));
