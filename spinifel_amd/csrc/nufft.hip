@@ -355,9 +355,12 @@ __device__ __forceinline__ void taps_pair_direct(__amdgpu_buffer_rsrc_t rsrc, in
 // took three barriers a tile instead of about one and a half: M = 121, 1,024 x 16k
 // points 1,830 us, now 1,550; 10k x 12.4k points 12.4 ms, now 10.7.  TP = 256 is one
 // tile a trip either way.  More staging loads in flight, running quotients for the
-// chunk addresses and 24-bit products all spill at 168 registers and lose.
+// chunk addresses and 24-bit products all spill at 168 registers and lose.  Kernels of 8 to
+// 12 points have two workgroups a CU and 256 registers: three spill up to 1,700 of theirs
+// (1,500 x 16k points, M = 81: W = 9, TP = 128 6.80 -> 4.13 ms, W = 10 17.1 -> 6.0, TP = 256
+// 10.8 -> 7.7); wider ones spill either way and gain more by the third (W = 13 18.6 and 21.8).
 template <int W, int TP>
-__global__ __launch_bounds__(256, 3) void k_slices_lds(GridView gv, const double *__restrict__ quats,
+__global__ __launch_bounds__(256, W >= 8 && W <= 12 ? 2 : 3) void k_slices_lds(GridView gv, const double *__restrict__ quats,
                                                     const double *__restrict__ q, int64_t N_p,
                                                     const int32_t *__restrict__ order,
                                                     int64_t n_order,
