@@ -172,11 +172,15 @@ class _Regulariser:
     """irfftn(rfftn(s . u) * mask) on M^3 values.  Odd M: axis by axis on complex
     transforms -- the values of the real ones bit for bit (odd lengths run as
     complex ones there too) without their copies between the axes (M = 81: 84
-    -> 60 us)."""
+    -> 60 us).  They take more calls, which up to M = 51 are the bound unless the
+    library's transforms are slow, by a factor above 17 (100 iterations, M = 17: 19.3
+    ms, 19.7 this way; 51 22.9 and 23.1; 41 36.9 and 35.5; 63 25.4 and 24.1)."""
 
     def __init__(self, lib, M, mask):
         self.lib, self.M, self.mask = lib, M, mask
-        self.odd = M % 2 == 1
+        factor = max((p for p in range(2, M + 1) if M % p == 0 and all(p % d for d in range(2, p))),
+                     default=1)
+        self.odd = M % 2 == 1 and (M > 52 or factor > 17)
         if self.odd:
             self.mask = mask.permute(2, 0, 1).contiguous()
             self.full = torch.empty((M,) * 3, dtype=torch.complex128, device=mask.device)
@@ -196,11 +200,12 @@ class _Regulariser:
         _lib.check(lib.mtip_half_expand(P(Z), M, P(self.full), st), "mtip_half_expand")
         return torch.fft.ifft(self.full, dim=2, norm="forward")
 
-    def values(self, u, support):
+    def values(self, u, support, product):
+        """product: s . u as (M, M, M)."""
         M = self.M
         if self.odd:
             return (self._back(u, support).real * (1.0 / M ** 3)).contiguous()
-        R = torch.fft.rfftn(u.view(M, M, M) * support)
+        R = torch.fft.rfftn(product)
         R *= self.mask
         return torch.fft.irfftn(R, s=(M, M, M)).contiguous()
 
@@ -208,7 +213,8 @@ class _Regulariser:
         """out += flambda s . values."""
         M, n = self.M, self.M ** 3
         if not self.odd:
-            out.view(M, M, M).addcmul_(self.values(u, support), support, value=flambda)
+            y = self.values(u, support, u.view(M, M, M) * support)
+            out.view(M, M, M).addcmul_(y, support, value=flambda)
             return
         P = engine._ptr
         _lib.check(self.lib.mtip_merge_reg_add(P(self._back(u, support)), 1.0 / n, P(support), flambda,
@@ -356,7 +362,7 @@ class Merge:
             X = torch.fft.rfftn(self._ups)
             X *= F_half
             y_ups = torch.fft.irfftn(X, s=(Mu,) * 3).contiguous()
-            y_reg = reg.values(u, sup)
+            y_reg = reg.values(u, sup, self._us)
             out = torch.empty(M ** 3, dtype=torch.float64, device=self.device)
             _lib.check(lib.mtip_merge_combine(P(y_ups), P(y_reg), P(u), P(sup), M, Mu,
                                               float(self.rlambda), float(self.flambda), P(out),

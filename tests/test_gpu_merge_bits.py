@@ -78,6 +78,26 @@ def test_operator_gives_the_bits_of_the_real_transforms(M, Mu):
         assert torch.equal(W(u), want)
 
 
+# complex transforms from 53 on and for factors above 17, real ones otherwise
+@pytest.mark.parametrize("M", [3, 17, 19, 37, 49, 51, 53, 55])
+def test_regulariser_on_both_sides_of_its_rule(M):
+    import torch
+    from spinifel_amd import _lib, engine, merge
+    engine.require_gpu()
+    print(f"case: M={M}", flush=True)
+    g = torch.Generator().manual_seed(M)
+    u = torch.randn(M ** 3, generator=g, dtype=torch.float64).cuda()
+    sup = (torch.rand((M,) * 3, generator=g) < 0.7).double().cuda()
+    mask = torch.rand((M, M, M // 2 + 1), generator=g, dtype=torch.float64).cuda()
+    us = u.view(M, M, M) * sup
+    R = torch.fft.rfftn(us)
+    R *= mask
+    want = torch.fft.irfftn(R, s=(M,) * 3)
+    reg = merge._Regulariser(_lib.load(), M, mask)
+    for _ in range(2):
+        assert torch.equal(reg.values(u, sup, us), want)
+
+
 if __name__ == "__main__":
     import sys
     np.savez_compressed(sys.argv[1], **{f"ac_{M}_{Mu}": _solve(M, Mu) for M, Mu in SIZES})
