@@ -364,7 +364,7 @@ __global__ __launch_bounds__(256, 3) void k_spread(GridView gv, double *__restri
 // or the data term to 1e-4 and more of the result, so another order of the sums
 // here changes what every merge returns (by up to 6e-9 where M = 9 and every spread
 // is one workgroup, so that runs give the same bits; at M = 81 two runs of one
-// program already differ by 1e-5 to 9e-4, through the order of the spread's atomics).
+// program already differ by 1e-5 to 2e-3, through the order of the spread's atomics).
 // Bound: a read of the table in LDS per product (M = 41 171 us, DFT matrices 29; M = 81
 // 317 and 68; M = 162 1,945 and 540).
 template <int MODE>

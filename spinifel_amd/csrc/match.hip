@@ -579,7 +579,7 @@ __global__ __launch_bounds__(512) void k_gemm_big(const uint8_t *__restrict__ A,
 // 6 / 16 of the FP32 product's time, and a sum takes 6 roundings per 16 pixels
 // instead of 16: the error against 64 bits is 0.6 - 0.9 of the FP32 instructions'
 // (16 to 16,384 pixels, normal, uniform and centred photon data; equal on data
-// of a wide range).  10,000 x 10,000 x 16,384: 26.8 -> 16.2 ms.
+// of a wide range).  10,000 x 10,000 x 16,384: 26.7 -> 15.4 ms.
 //
 // The three parts are exact from 2^-110 up to where a bf16 rounds to infinity.  A sum
 // that is not finite (an infinity or a NaN in an operand, a value that rounds to one, a
