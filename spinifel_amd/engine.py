@@ -183,6 +183,12 @@ def _orient_rank(quats):
     return rank
 
 
+def _slots(det_shape, edge):
+    """Slots of a detector in edge x edge blocks, padding included."""
+    rows, cols = det_shape[-2:]
+    return math.prod(det_shape[:-2]) * -(-rows // edge) * -(-cols // edge) * edge * edge
+
+
 def auto_tiling(plan, det_shape):
     """Tiling by rule, without timing: 16 x 16 blocks while a block's fine-grid
     box fits LDS, which takes pixels no further apart than about 1.4 cells of
@@ -195,16 +201,26 @@ def auto_tiling(plan, det_shape):
     every grid up to 200 points (2,000 of 32 x 32, n = 90, 4 points: 159 us for
     8 x 8, 123 for 16 x 16; of 64 x 64, n = 180: 522 and 507), at 5 points up to 100
     or twice the edge (n = 90: 183 and 168; 90 x 90, n = 162: 1,000 and 790; 64 x
-    64, n = 162: 564 and 636).  The autotuner (spinifel_amd.autotune) picks by timing."""
-    if len(tuple(det_shape)) < 2:
+    64, n = 162: 564 and 636).  Kernels of 13 points and more spill most with 64-point
+    tiles: 16 x 16 wins on grids of up to 200 points (500 of 90 x 90, n = 162, 13
+    points: 8,590 us for 8 x 8, 4,090 for 16 x 16; of 12 x 9, n = 30: 278 and 145) unless
+    8 x 8 leaves a quarter less padding (24 x 20, n = 90, 14 points: 0.80 of the
+    time).  A detector of one 16 x 16 block, not of a smaller one, has as many points a
+    trip either way (15 of 16 x 16, n = 50, 7 points: 46.6 and 38.7).  The autotuner
+    (spinifel_amd.autotune) picks by timing."""
+    det_shape = tuple(int(d) for d in det_shape)
+    if len(det_shape) < 2:
         return None
-    edge = math.sqrt(math.prod(int(d) for d in det_shape))
+    edge = math.sqrt(math.prod(det_shape))
+    slots8, slots16 = _slots(det_shape, 8), _slots(det_shape, 16)
     width = getattr(plan, "width", 7)
     most = 1.6 * edge
-    if width <= 4:
+    if width <= 4 or (width <= 7 and slots8 == slots16 == 256):
         most = max(most, 200)
     elif width == 5:
         most = max(most, 100, min(200, 2 * edge))
+    elif width >= 13 and 4 * slots8 > 3 * slots16:
+        most = max(most, 200)
     return tiling(det_shape, (16, 16) if plan.n_fine <= most else (8, 8))
 
 
